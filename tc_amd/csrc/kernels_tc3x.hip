@@ -161,50 +161,43 @@ void launch_products_fft(int prec, const PairEntry* pairs, int npairs, const Pro
     launch_fft_xy(prec, -1, out, npairs * nchan, g, s);
 }
 
-// ----------------------------------------------------------------- tc3a3b3b4b6
-// out[j][d](r) = dnu_d(r) * phi_j(r) in the working precision (dnu FP64, 3 grids)
+// [3a3] (tc3a3b3b4b6.cpp:629-642): W[j] += fa3 sum_d qsum[j][d] dnu_d, and the source field of
+// phase 2, v[j][d] = qsum[j][d] + b34 dnu_d phi_j in the working precision: [3b3] (:284-303) and
+// [3b4] (:740-754) apply the same map sum_q f phi_q FFT_backward(sum_d du_0,d FFT_forward(conj(chi_q) .))
+// to b3 dnu_d phi_j and to b4 qsum_j,d, so with b34 = b3/b4 one pass over the pairs serves both.
+// Before, [3b3] carried three record channels and an output of its own through phase 1 (36 grids
+// of traffic per pair there, now 28): tc3a3b3b4b6 at 40^3, 2x2x2 k, 12 bands, FP32 59.9 -> 50.1 ms;
+// 30^3 FP64 7.9 -> 6.5 ms.
 template <typename T>
-__global__ __launch_bounds__(256) void k_mul_dnu(const cpx<T>* __restrict__ appR, const double2* __restrict__ dnu,
-                                                 cpx<T>* __restrict__ out, int j0, long long N)
+__global__ __launch_bounds__(256) void k_a3_b34(double2* __restrict__ W, const double2* __restrict__ qsum,
+                                                const double2* __restrict__ dnu, const cpx<T>* __restrict__ appR,
+                                                cpx<T>* __restrict__ v, int j0, long long N, double fa3, double b34)
 {
     const long long r = (long long)blockIdx.x * 256 + threadIdx.x;
     if (r >= N) return;
     const int j = j0 + (int)blockIdx.y;
-    const double2 ph = up(appR[(long long)j * N + r]);
-    for (int d = 0; d < 3; ++d) out[((long long)j * 3 + d) * N + r] = down<T>(dmul(dnu[(long long)d * N + r], ph));
-}
-
-void launch_mul_dnu(int prec, const void* appR, const double* dnu, void* out, int napp, long long N, hipStream_t s)
-{
-    for_slices(napp, [&](int j0, unsigned ny) {
-        if (prec == TCX_PREC_FP64)
-            hipLaunchKernelGGL(k_mul_dnu<double>, grid_pts(N, ny), dim3(256), 0, s, (const cpx<double>*)appR,
-                               (const double2*)dnu, (cpx<double>*)out, j0, N);
-        else
-            hipLaunchKernelGGL(k_mul_dnu<float>, grid_pts(N, ny), dim3(256), 0, s, (const cpx<float>*)appR,
-                               (const double2*)dnu, (cpx<float>*)out, j0, N);
-        TCX_HIP_CHECK(hipGetLastError());
-    });
-}
-
-// [3a3] (tc3a3b3b4b6.cpp:629-642): W[j] += fa3 sum_d qsum[j][d] dnu_d
-__global__ __launch_bounds__(256) void k_a3(double2* __restrict__ W, const double2* __restrict__ qsum,
-                                            const double2* __restrict__ dnu, int j0, long long N, double fa3)
-{
-    const long long r = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (r >= N) return;
-    const int j = j0 + (int)blockIdx.y;
+    const double2 ph = dscale(up(appR[(long long)j * N + r]), b34);
     double2 acc = make_double2(0.0, 0.0);
-    for (int d = 0; d < 3; ++d) acc = dadd(acc, dmul(qsum[((long long)j * 3 + d) * N + r], dnu[(long long)d * N + r]));
+    for (int d = 0; d < 3; ++d) {
+        const long long o = ((long long)j * 3 + d) * N + r;
+        const double2 q = qsum[o], n = dnu[(long long)d * N + r];
+        acc = dadd(acc, dmul(q, n));
+        v[o] = down<T>(dadd(q, dmul(n, ph)));
+    }
     double2* w = W + (long long)j * N + r;
     *w = dadd(*w, dscale(acc, fa3));
 }
 
-void launch_a3(double* W, const double* qsum, const double* dnu, int napp, long long N, double fa3, hipStream_t s)
+void launch_a3_b34(int prec, double* W, const double* qsum, const double* dnu, const void* appR, void* v, int napp,
+                   long long N, double fa3, double b34, hipStream_t s)
 {
     for_slices(napp, [&](int j0, unsigned ny) {
-        hipLaunchKernelGGL(k_a3, grid_pts(N, ny), dim3(256), 0, s, (double2*)W, (const double2*)qsum,
-                           (const double2*)dnu, j0, N, fa3);
+        if (prec == TCX_PREC_FP64)
+            hipLaunchKernelGGL(k_a3_b34<double>, grid_pts(N, ny), dim3(256), 0, s, (double2*)W, (const double2*)qsum,
+                               (const double2*)dnu, (const cpx<double>*)appR, (cpx<double>*)v, j0, N, fa3, b34);
+        else
+            hipLaunchKernelGGL(k_a3_b34<float>, grid_pts(N, ny), dim3(256), 0, s, (double2*)W, (const double2*)qsum,
+                               (const double2*)dnu, (const cpx<float>*)appR, (cpx<float>*)v, j0, N, fa3, b34);
         TCX_HIP_CHECK(hipGetLastError());
     });
 }

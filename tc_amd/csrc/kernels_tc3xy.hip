@@ -12,8 +12,8 @@
 // and the rest skip it; the du_s,d outputs leave in rounds of their three d components.
 // The combines are the reference's G-space products with
 // du_s,d(G) = (kq+G)_d u(kq+G, s):
-//   tc3a3b3b4b6 (src/calc_hamiltonian_tc3a3b3b4b6.cpp): [3b3] and the [3a3,b4,b6] channels
-//     (:280-349), the [3b3]+[3b6] merge (:344-358), [3b4] (:740-754);
+//   tc3a3b3b4b6 (src/calc_hamiltonian_tc3a3b3b4b6.cpp): the [3a3,b4,b6] channels (:305-343), the
+//     [3b6] sum (:344-358), [3b3] and [3b4] as one (:284-303, :740-754);
 //   tc3a2a4b2b5 (src/calc_hamiltonian_tc3a2a4b2b5.cpp): the q1-q2 channels (:371-375) and
 //     the apply-phase channels (:849-876).
 // u(kq+G, s) comes from a per-launch table (FP64 evaluation rounded once to the working
@@ -199,8 +199,8 @@ constexpr int tiles_a7c2()
 
 // Tiles per workgroup of each pass: as many as its largest group of channels transformed
 // together (three tiles give 4 workgroups of 2 wavefronts per CU at 40^3 in FP32, four
-// tiles 3 of 3).  a7c1 transforms its four inputs as three, then one.
-constexpr int kTilesA7c1 = 3, kTilesB4 = 3, kTilesA8c1 = 3;
+// tiles 3 of 3).
+constexpr int kTilesB4 = 3, kTilesA8c1 = 3;
 
 // a8c2 transforms its four inputs at once in FP32 and as three, then one, in FP64 (at 40^3
 // two workgroups of 2 wavefronts per CU against one of 3): tc3a2a4b2b5 at 40^3 took 6.59 s
@@ -233,57 +233,9 @@ __global__ __launch_bounds__(256) void k_u2_table(cpx<T>* __restrict__ tab, cons
 }
 
 // ----------------------------------------------------------------- tc3a3b3b4b6
-// Phase-1 combine.  In: rec[p][0..3] = z-transformed (conj(chi_qi) phi_j, conj(chi_qi) dnu_d phi_j).
-// Out: Y[p] = f b3 sum_d du_0,d rec[p][1+d] in G space (completed later by the second combine);
-//      P[p][3s+d] = f du_s,d rec[p][0], inverse-transformed along x and y.
-template <typename T, int NP>
-__global__ __launch_bounds__((XyGroup<NP, kTilesA7c1>::threads))
-void k_xy_a7c1(
-    const cpx<T>* __restrict__ rec, cpx<T>* __restrict__ P, cpx<T>* __restrict__ Y, const PairEntry* __restrict__ pairs,
-    const cpx<T>* __restrict__ tab, int kq0, const double* __restrict__ kqcart, const double* __restrict__ fill, int nz,
-    Geom g, double fb3)
-{
-    constexpr int NT = kTilesA7c1;
-    constexpr int EPT = XyGroup<NP, NT>::ept;
-    __shared__ XyTiles<T, NP, NT> S;
-    const XyLane<NP, NT> L;
-    const int z = blockIdx.x, p = blockIdx.y;
-    const size_t ng = (size_t)NP * NP * nz, pz = (size_t)z * NP * NP;
-    const PairEntry pe = pairs[p];
-    const PlanePoint pp(kqcart + 3 * pe.kq, g, z, nz);
-    const cpx<T>* tp = tab + (size_t)(pe.kq - kq0) * ng + pz;
-    const double f = fill[pe.occ];
-    cpx<T> u[EPT];
-    load_points<T, NP, NT>(u, tp);
-    // rec[p][1+d] in tiles d -> Y; then rec[p][0] in tile 0, kept in registers
-    xy_forward<T, NP>(S.t[L.tile()], rec + ((size_t)p * 4 + 1 + L.tile()) * ng + pz, L.c < 3, L.t);
-    for_points<NP, NT>([&](auto ic, int e, int x, int y) {
-        constexpr int i = decltype(ic)::value;
-        double xd[3];
-        pp.at(g, x, y, NP, xd);
-        const double u0 = (double)u[i].re;
-        double2 acc = make_double2(0.0, 0.0);
-        for (int d = 0; d < 3; ++d) {
-            const double2 s = up2(S.t[d].a[y][x]);
-            acc.x += s.x * (xd[d] * u0);
-            acc.y += s.y * (xd[d] * u0);
-        }
-        Y[(size_t)p * ng + pz + e] = down2<T>(make_double2(acc.x * (f * fb3), acc.y * (f * fb3)));
-    });
-    __syncthreads();  // the tiles have been read before rec[p][0] overwrites tile 0
-    xy_forward<T, NP>(S.t[0], rec + (size_t)p * 4 * ng + pz, L.c == 0, L.t);
-    cpx<T> r0[EPT];
-    for_points<NP, NT>([&](auto ic, int e, int x, int y) { r0[decltype(ic)::value] = S.t[0].a[y][x]; });
-    __syncthreads();  // the input has been read before outputs overwrite the tiles
-    xy_du_rounds<T, NP, NT, 2>(
-        S, pp, g, u, [&](auto ic, int) { return r0[decltype(ic)::value]; },
-        [&](int k, cpx<T> uk) { return f * (double)(k == 0 ? uk.re : uk.im); },
-        [&](int o) { return P + ((size_t)p * 6 + o) * ng + pz; });
-}
-
-// Phase-1 second combine ([3b3] and [3b6] merged by linearity).  In: P[p][0..5] z-transformed
-// (after the density step), Y[p] in G space.  Out: Y[p] += b6 sum_{s,d} du_s,d P[p][3s+d],
-// inverse-transformed along x and y (in place).
+// Phase-1 combine after the density step ([3b6]).  In: P[p][0..5] z-transformed.  Out: Y[p] =
+// b6 sum_{s,d} du_s,d P[p][3s+d], inverse-transformed along x and y.  The channels before the
+// density step are k_xy_a8c1's (du_s,d rho), without the filling: the consumers weight by it.
 template <typename T, int NP>
 __global__ __launch_bounds__((XyGroup<NP, tiles_a7c2<T, NP>()>::threads))
 void k_xy_a7c2(
@@ -299,9 +251,8 @@ void k_xy_a7c2(
     const PairEntry pe = pairs[p];
     const PlanePoint pp(kqcart + 3 * pe.kq, g, z, nz);
     const cpx<T>* tp = tab + (size_t)(pe.kq - kq0) * ng + pz;
-    cpx<T> u[EPT], yv[EPT];
+    cpx<T> u[EPT];
     load_points<T, NP, NT>(u, tp);
-    load_points<T, NP, NT>(yv, Y + (size_t)p * ng + pz);
     if constexpr (NT == 6) {
         // all six channels at once: channel 3s + d in tile 3s + d
         xy_forward<T, NP>(S.t[L.tile()], P + ((size_t)p * 6 + L.tile()) * ng + pz, L.c < 6, L.t);
@@ -309,7 +260,7 @@ void k_xy_a7c2(
             constexpr int i = decltype(ic)::value;
             double xd[3];
             pp.at(g, x, y, NP, xd);
-            double2 a = up2(yv[i]);
+            double2 a = make_double2(0.0, 0.0);
             for (int sp = 0; sp < 2; ++sp) {
                 const double us = fb6 * (double)(sp == 0 ? u[i].re : u[i].im);
                 for (int d = 0; d < 3; ++d) {
@@ -332,7 +283,7 @@ void k_xy_a7c2(
                 double xd[3];
                 pp.at(g, x, y, NP, xd);
                 const double us = fb6 * (double)(sp == 0 ? u[i].re : u[i].im);
-                double2 a = sp == 0 ? up2(yv[i]) : acc[i];
+                double2 a = sp == 0 ? make_double2(0.0, 0.0) : acc[i];
                 for (int d = 0; d < 3; ++d) {
                     const double2 v = up2(S.t[d].a[y][x]);
                     a.x += v.x * (xd[d] * us);
@@ -349,7 +300,8 @@ void k_xy_a7c2(
     xy_inverse_store<T, NP>(S.t[0], Y + (size_t)p * ng + pz, L.c == 0, L.t);
 }
 
-// Phase-2 combine ([3b4]).  In: rec[p][0..2] z-transformed conj(chi_qi) qsum_j,d.
+// Phase-2 combine ([3b3] + [3b4]).  In: rec[p][0..2] z-transformed conj(chi_qi) v_j,d,
+// v_j,d = qsum_j,d + (b3 / b4) dnu_d phi_j.
 // Out: Z[p] = b4 f sum_d du_0,d rec[p][d], inverse-transformed along x and y.
 template <typename T, int NP>
 __global__ __launch_bounds__((XyGroup<NP, kTilesB4>::threads))
@@ -388,7 +340,7 @@ void k_xy_b4(
 }
 
 // ----------------------------------------------------------------- tc3a2a4b2b5
-// q1-q2 combine.  In: rec[p][h] z-transformed (h = 0: conj(chi_q1) phi_q2; BITC h = 1:
+// q1-q2 combine, and with one input the channels du_s,d rho of tc3a3b3b4b6 phase 1.  In: rec[p][h] z-transformed (h = 0: conj(chi_q1) phi_q2; BITC h = 1:
 // conj(phi_q1) chi_q2).  Out: O[p][6h + 3s + d] = du12_s,d rec[p][h], inverse-transformed
 // along x and y.  The NIN inputs are transformed side by side; each thread then keeps its
 // points of them in registers, so every tile can take outputs.
@@ -547,21 +499,6 @@ void launch_u2_table(int prec, void* tab, const double* kqcart, int row0, int nr
         }                                                     \
         TCX_HIP_CHECK(hipGetLastError());                     \
     } while (0)
-
-void launch_xy_a7c1(int prec, const Geom& g, const void* rec, void* P, void* Y, const PairEntry* pairs, int npairs,
-                    const void* tab, int kq0, const double* kqcart, const double* fill, double fb3, hipStream_t s)
-{
-    const size_t es = prec == TCX_PREC_FP64 ? 16 : 8, gb = (size_t)g.n1 * g.n2 * g.n3 * es;
-    for_pair_slices(npairs, [&](int a, int n) {
-#define TCX_L(NP)                                                                                               \
-    hipLaunchKernelGGL((k_xy_a7c1<T, NP>), dim3(g.n3, n), (xy_block<NP, kTilesA7c1>()), 0, s,                   \
-                       (const cpx<T>*)((const char*)rec + (size_t)a * 4 * gb),                                  \
-                       (cpx<T>*)((char*)P + (size_t)a * 6 * gb), (cpx<T>*)((char*)Y + (size_t)a * gb), pairs + a, \
-                       (const cpx<T>*)tab, kq0, kqcart, fill, g.n3, g, fb3);
-        TCX_XY_DISPATCH(prec, g, TCX_L);
-#undef TCX_L
-    });
-}
 
 void launch_xy_a7c2(int prec, const Geom& g, const void* P, void* Y, const PairEntry* pairs, int npairs,
                     const void* tab, int kq0, const double* kqcart, double fb6, hipStream_t s)

@@ -7,7 +7,7 @@
 // applies the consumer at the lane's output points, summing in FP64 registers, and adds
 // once into the FP64 grids of the target (no atomics, deterministic).  The consumers are
 // the reference's real-space steps:
-//   tc3a3b3b4b6 (src/calc_hamiltonian_tc3a3b3b4b6.cpp:316-335): qsum_j,d += P_0,d phi_qi,
+//   tc3a3b3b4b6 (src/calc_hamiltonian_tc3a3b3b4b6.cpp:316-335): qsum_j,d += f P_0,d phi_qi,
 //     then P_s,d *= density_s, transformed along z again for the next FFT_forward;
 //   tc3a2a4b2b5 (src/calc_hamiltonian_tc3a2a4b2b5.cpp:377-427): the q-sums Q2, Q4, Q5;
 //     (:848-913) the apply-phase accumulation into W.
@@ -61,7 +61,7 @@ __device__ __forceinline__ void zinv(cpx<T> (&v)[NZ / S], const cpx<T>* grid, co
 }  // namespace
 
 // ----------------------------------------------------------------- tc3a3b3b4b6 real-space step
-// Per target (k,j) and direction d = blockIdx.z: qsum[j][d] += sum_p P[p][d] phi_qi (the
+// Per target (k,j) and direction d = blockIdx.z: qsum[j][d] += sum_p f P[p][d] phi_qi (the
 // s2 = 0 channel, before the density), and P[p][3s+d] <- FFT_z(density_s * P[p][3s+d]) * sc
 // for s = 0, 1 (in place): the real-space step between the z pass of FFT_backward and the
 // z pass of the next FFT_forward.  The lanes of a pencil move from the blocked output layout
@@ -70,6 +70,7 @@ template <typename T, int NZ, int S>
 __global__ __launch_bounds__(kPencilBlock) void k_za7_mid(cpx<T>* __restrict__ P, const cpx<T>* __restrict__ occR,
                                                           const PairEntry* __restrict__ pairs,
                                                           const TargetEntry* __restrict__ targets,
+                                                          const double* __restrict__ fill,
                                                           const double2* __restrict__ dens, size_t dstride,
                                                           double2* __restrict__ qsum, int nxy, T sc)
 {
@@ -94,7 +95,9 @@ __global__ __launch_bounds__(kPencilBlock) void k_za7_mid(cpx<T>* __restrict__ P
 #pragma unroll 1
     for (int it = 0; it < nsteps; ++it) {
         const int pp = te.pair0 + (it >> 1), s = it & 1;
-        const cpx<T>* ph = occR + (size_t)pairs[pp].occ * ng + o0;
+        const int occ = pairs[pp].occ;
+        const double f = fill[occ];
+        const cpx<T>* ph = occR + (size_t)occ * ng + o0;
         cpx<T>* g = grid_of(it);
         cpx<T> v[M];
         if (kPrefetch) {
@@ -122,10 +125,10 @@ __global__ __launch_bounds__(kPencilBlock) void k_za7_mid(cpx<T>* __restrict__ P
                 const double2 x = upd(v[k]);
                 double2 dn;
                 if constexpr (kPrefetch) {
-                    if (s == 0) acc[k] = cmadd(acc[k], x, upd(phv[k]), 1.0);
+                    if (s == 0) acc[k] = cmadd(acc[k], x, upd(phv[k]), f);
                     dn = dnv[k];
                 } else {
-                    if (s == 0) acc[k] = cmadd(acc[k], x, upd(ph[(size_t)k * nxy]), 1.0);
+                    if (s == 0) acc[k] = cmadd(acc[k], x, upd(ph[(size_t)k * nxy]), f);
                     dn = n[(size_t)k * nxy];
                 }
                 xs[pi][L.ob * M + k] = cpx<T>{(T)(x.x * dn.x - x.y * dn.y), (T)(x.x * dn.y + x.y * dn.x)};
@@ -368,8 +371,8 @@ void for_target_slices(int n, F&& f)
     } while (0)
 
 void launch_za7_mid(int prec, const Geom& g, void* P, const void* occR, const PairEntry* pairs,
-                    const TargetEntry* targets, int ntargets, const double* dens, long long dens_stride,
-                    double* qsum, double sc, hipStream_t s)
+                    const TargetEntry* targets, int ntargets, const double* fill, const double* dens,
+                    long long dens_stride, double* qsum, double sc, hipStream_t s)
 {
     const int nxy = g.n1 * g.n2;
     for_target_slices(ntargets, [&](int a, int n) {
@@ -378,7 +381,7 @@ void launch_za7_mid(int prec, const Geom& g, void* P, const void* occR, const Pa
         constexpr int S = SplitFor<NZ, 4>::value;                                                            \
         constexpr int PN = PencilSplit<S>::pencils;                                                          \
         hipLaunchKernelGGL((k_za7_mid<T, NZ, S>), dim3((nxy + PN - 1) / PN, n, 3), dim3(kPencilBlock), 0, s,\
-                           (cpx<T>*)P, (const cpx<T>*)occR, pairs, targets + a, (const double2*)dens,        \
+                           (cpx<T>*)P, (const cpx<T>*)occR, pairs, targets + a, fill, (const double2*)dens,  \
                            (size_t)dens_stride, (double2*)qsum, nxy, (T)sc);                                 \
     }
         TCX_Z_DISPATCH(prec, g, TCX_L);

@@ -182,8 +182,6 @@ void launch_products_z(int prec, const PairEntry* pairs, int npairs, const ProdC
 // (u(kq+G, j0), u(kq+G, j1)) per k-q row of the launch (launch_u2_table)
 void launch_u2_table(int prec, void* tab, const double* kqcart, int row0, int nrows, const Geom& g,
                      const JastrowPair& j0, const JastrowPair& j1, hipStream_t s);
-void launch_xy_a7c1(int prec, const Geom& g, const void* rec, void* P, void* Y, const PairEntry* pairs, int npairs,
-                    const void* tab, int kq0, const double* kqcart, const double* fill, double fb3, hipStream_t s);
 void launch_xy_a7c2(int prec, const Geom& g, const void* P, void* Y, const PairEntry* pairs, int npairs,
                     const void* tab, int kq0, const double* kqcart, double fb6, hipStream_t s);
 void launch_xy_b4(int prec, const Geom& g, const void* rec, void* Z, const PairEntry* pairs, int npairs,
@@ -196,16 +194,16 @@ void launch_xy_a8c2(int prec, const Geom& g, const void* rec, void* Z, const Pai
 // z passes of FFT_backward fused with the real-space consumers (kernels_tc3z.hip)
 // dens_stride: complex elements between the two spin densities (0: one independent spin)
 void launch_za7_mid(int prec, const Geom& g, void* P, const void* occR, const PairEntry* pairs,
-                    const TargetEntry* targets, int ntargets, const double* dens, long long dens_stride,
-                    double* qsum, double sc, hipStream_t s);
+                    const TargetEntry* targets, int ntargets, const double* fill, const double* dens,
+                    long long dens_stride, double* qsum, double sc, hipStream_t s);
 void launch_za8_q(int prec, const Geom& g, const void* O, int bitc, const void* occR, const void* chiR,
                   const PairEntry* pairs, const TargetEntry* targets, int ntargets, const double* fill, double* Q2,
                   double* Q4, double* Q5, hipStream_t s);
 void launch_za8_apply(int prec, const Geom& g, const void* Z, const void* occR, const void* Q4T,
                       const PairEntry* pairs, const TargetEntry* targets, int ntargets, double* W, float* Wc,
                       hipStream_t s);
-void launch_mul_dnu(int prec, const void* appR, const double* dnu, void* out, int napp, long long N, hipStream_t s);
-void launch_a3(double* W, const double* qsum, const double* dnu, int napp, long long N, double fa3, hipStream_t s);
+void launch_a3_b34(int prec, double* W, const double* qsum, const double* dnu, const void* appR, void* v, int napp,
+                   long long N, double fa3, double b34, hipStream_t s);
 void launch_b6(const double* nG, double* tG, double* t1, const double* dcp, const int* match, int nk, const Geom& g,
                long long N,
                const JastrowPair& j0, const JastrowPair& j1, hipStream_t s);

@@ -132,11 +132,9 @@ void Context::tc3a3b3b4b6(const int* nb_, const double* phi, double* out, int pr
         launch_dnu(nG, dnu, geo, j00, j01, stream);
         launch_fft3d(TCX_PREC_FP64, +1, dnu, 3, geo, 1.0, stream);
 
-        // applied orbitals and dnu_d phi_j in real space
+        // applied orbitals in real space
         d_appR.ensure((size_t)P.n_app * gT);
-        d_appGrad.ensure((size_t)3 * P.n_app * gT);
         orbitals_to_real(io.phi, (const OrbEntry*)P.d_appjobs.p, P.n_app, prec, d_appR.p);
-        launch_mul_dnu(prec, d_appR.p, dnu, d_appGrad.p, P.n_app, N, stream);
 
         begin_W(P.n_app);
         d_qsum.ensure((size_t)3 * P.n_app * g64);
@@ -144,42 +142,39 @@ void Context::tc3a3b3b4b6(const int* nb_, const double* phi, double* out, int pr
         double* W = (double*)d_W.p;
         double* qsum = (double*)d_qsum.p;
 
-        const PairSet& S = pair_set(nb, kPairsAppOcc, 11, prec);
-        d_rec.ensure((size_t)std::max(1, S.max_launch_pairs) * 11 * gT);
+        const PairSet& S = pair_set(nb, kPairsAppOcc, 7, prec);  // rho and six channels
+        d_rec.ensure((size_t)std::max(1, S.max_launch_pairs) * 7 * gT);
         const double* kq = (const double*)S.d_kq.p;
         int max_rows = 1;
         for (const Launch& L : S.launches) max_rows = std::max(max_rows, L.nkq);
         d_ktab.ensure((size_t)max_rows * gT);  // (u(kq+G, 00), u(kq+G, 10)) per k-q row
         const double* fill = (const double*)d_fill.p;
 
-        // phase 1: [3b3], [3a3,b4,b6] (:179-371)
+        // phase 1: [3a3,b4,b6] (:179-371); [3b3] joins [3b4] in phase 2
         {
-            ProdChan ch[4];
-            ch[0] = chan(chiR, 1, 1, 0, 1, d_appR.p, 0, 1, 0, 0);
-            for (int d = 0; d < 3; ++d) ch[1 + d] = chan(chiR, 1, 1, 0, 1, d_appGrad.p, 0, 3, d, 0);
-            upload(d_chans, ch, sizeof(ch));
+            const ProdChan ch = chan(chiR, 1, 1, 0, 1, d_appR.p, 0, 1, 0, 0);
+            upload(d_chans, &ch, sizeof(ch));
         }
         for (const Launch& L : S.launches) {
             const PairEntry* pairs = (const PairEntry*)S.d_pairs.p + L.pair0;
             const TargetEntry* targets = (const TargetEntry*)S.d_targets.p + L.target0;
             const int np = L.npairs;
-            char* rec4 = (char*)d_rec.p;
-            char* Pb = rec4 + (size_t)4 * np * gT;
-            char* Y = Pb + (size_t)6 * np * gT;
+            char* rec = (char*)d_rec.p;
+            char* Pb = rec + (size_t)np * gT;
+            char* Y = rec;  // rho has been read when Y is formed
             launch_u2_table(prec, d_ktab.p, kq, L.kq0, L.nkq, geo, j00, j10, stream);
             timed(0, np, [&] {
-                launch_products_z(prec, pairs, np, (const ProdChan*)d_chans.p, 4, rec4, geo, 1.0 / (double)N,
-                                  stream);
+                launch_products_z(prec, pairs, np, (const ProdChan*)d_chans.p, 1, rec, geo, 1.0 / (double)N, stream);
             });
             timed(1, np, [&] {
-                launch_xy_a7c1(prec, geo, rec4, Pb, Y, pairs, np, d_ktab.p, L.kq0, kq, fill, fb3, stream);
+                launch_xy_a8c1(prec, geo, rec, 1, Pb, pairs, np, d_ktab.p, L.kq0, kq, stream);
                 // one independent spin: both spin channels read the one density grid
-                launch_za7_mid(prec, geo, Pb, occR, pairs, targets, L.ntargets, (const double*)d_density.p,
+                launch_za7_mid(prec, geo, Pb, occR, pairs, targets, L.ntargets, fill, (const double*)d_density.p,
                                nspin == 1 ? 0 : N, qsum, 1.0 / (double)N, stream);
                 launch_xy_a7c2(prec, geo, Pb, Y, pairs, np, d_ktab.p, L.kq0, kq, fb6, stream);
             });
             timed(2, np, [&] {  // z pass of FFT_backward fused with the accumulation
-                launch_hf2x_C(prec, geo, Y, occR, pairs, targets, L.ntargets, nullptr, W, (float*)d_Wc.p, stream);
+                launch_hf2x_C(prec, geo, Y, occR, pairs, targets, L.ntargets, fill, W, (float*)d_Wc.p, stream);
             });
         }
 
@@ -248,19 +243,14 @@ void Context::tc3a3b3b4b6(const int* nb_, const double* phi, double* out, int pr
                 }
             }
         }
-        // [3a3] (:629-642)
-        launch_a3(W, qsum, dnu, P.n_app, N, fa3, stream);
+        // [3a3] (:629-642) and the source field of phase 2
+        d_qsumT.ensure((size_t)3 * P.n_app * gT);
+        launch_a3_b34(prec, W, qsum, dnu, d_appR.p, d_qsumT.p, P.n_app, N, fa3, fb3 / fb4, stream);
 
-        // phase 2: [3b4] (:646-770), products conj(chi_qi) qsum_j,d in the working precision
-        const void* qsumT = qsum;
-        if (prec == TCX_PREC_FP32) {
-            d_qsumT.ensure((size_t)3 * P.n_app * gT);
-            launch_convert_d2f(qsum, (float*)d_qsumT.p, (long long)3 * P.n_app * N, stream);
-            qsumT = d_qsumT.p;
-        }
+        // phase 2: [3b3] (:284-303) and [3b4] (:646-770)
         {
             ProdChan ch[3];
-            for (int d = 0; d < 3; ++d) ch[d] = chan(chiR, 1, 1, 0, 1, qsumT, 0, 3, d, 0);
+            for (int d = 0; d < 3; ++d) ch[d] = chan(chiR, 1, 1, 0, 1, d_qsumT.p, 0, 3, d, 0);
             upload(d_chans, ch, sizeof(ch));
         }
         for (const Launch& L : S.launches) {
