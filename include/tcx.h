@@ -383,9 +383,9 @@ int tcx_memset_zero(tcx_context *ctx, void *ptr, unsigned long long bytes);
 /* Pass order of the exchange pair pipeline (term 0: hf2x): 0 z-first (transform along z,
  * then the xy planes, then z back), 1 plane-first (xy planes, then z pencils, then xy back;
  * FP32-split only: the pair records then hold only the (kx, ky) columns inside the pair
- * density's G-space support, about two thirds of them at 40^3), -1 automatic (z-first;
- * the default: plane-first moves fewer bytes but ran slower at 40^3).  No counterpart in
- * the reference, whose hf2x runs full 3D FFTs (src/calc_hamiltonian_hf2x.cpp:123-135);
+ * density's G-space support, about two thirds of them at 40^3), -1 automatic (the default:
+ * plane-first in FP32-split, except in the applies of tcx_davidson).  No counterpart in the
+ * reference, whose hf2x runs full 3D FFTs (src/calc_hamiltonian_hf2x.cpp:123-135);
  * the two orders agree to rounding. */
 int tcx_set_pipeline_order(tcx_context *ctx, int term, int order);
 

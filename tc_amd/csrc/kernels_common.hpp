@@ -359,4 +359,62 @@ __device__ __forceinline__ void tile_get_row(const PlaneTile<T, NP>& s, cpx<T> (
     });
 }
 
+// LDS tile of one component (real or imaginary part) of a plane, [y][x] with one
+// element of padding per row.  FP64 passes transpose the two parts one after the other: that
+// halves their LDS per plane and doubles their waves per SIMD (1 -> 2 at 40^3, hf2x pass B).
+// FP32 keeps whole complex tiles: split tiles would double its waves too (2 -> 4), but with
+// twice the LDS instructions and three times the barriers the pass ran 5% slower.
+template <typename T, int NP>
+struct PartTile {
+    T a[NP][NP + 1];
+};
+template <typename T, int NP>
+using TransposeTile = std::conditional_t<sizeof(T) == 8, PartTile<T, NP>, PlaneTile<T, NP>>;
+template <int C, typename T>
+__device__ __forceinline__ T& part(cpx<T>& z)
+{
+    if constexpr (C == 0) return z.re; else return z.im;
+}
+
+// Transposes of the planes of a workgroup: an active thread turns its column x = col (values
+// along y) into row y = row (values along x), and back.  Every thread of the workgroup calls
+// them (they contain the barriers); no barrier before the first write, so the tile must have
+// been read by then, except that rows_to_cols may follow cols_to_rows with the same row.
+template <typename T, int NP>
+__device__ __forceinline__ void cols_to_rows(PlaneTile<T, NP>& s, cpx<T> (&v)[NP], int col, int row, bool active)
+{
+    if (active) tile_put_col<T, NP>(s, v, col);
+    __syncthreads();
+    if (active) tile_get_row<T, NP>(s, v, row);
+}
+template <typename T, int NP>
+__device__ __forceinline__ void rows_to_cols(PlaneTile<T, NP>& s, cpx<T> (&v)[NP], int row, int col, bool active)
+{
+    if (active) tile_put_row<T, NP>(s, v, row);  // that row was read by this thread alone
+    __syncthreads();
+    if (active) tile_get_col<T, NP>(s, v, col);
+}
+template <typename T, int NP>
+__device__ __forceinline__ void cols_to_rows(PartTile<T, NP>& s, cpx<T> (&v)[NP], int col, int row, bool active)
+{
+    static_for<0, 2>([&](auto cc) {
+        constexpr int C = decltype(cc)::value;
+        if constexpr (C == 1) __syncthreads();  // every thread has read the real parts
+        if (active) static_for<0, NP>([&](auto yc) { s.a[decltype(yc)::value][col] = part<C>(v[decltype(yc)::value]); });
+        __syncthreads();
+        if (active) static_for<0, NP>([&](auto xc) { part<C>(v[decltype(xc)::value]) = s.a[row][decltype(xc)::value]; });
+    });
+}
+template <typename T, int NP>
+__device__ __forceinline__ void rows_to_cols(PartTile<T, NP>& s, cpx<T> (&v)[NP], int row, int col, bool active)
+{
+    static_for<0, 2>([&](auto cc) {
+        constexpr int C = decltype(cc)::value;
+        if constexpr (C == 1) __syncthreads();
+        if (active) static_for<0, NP>([&](auto xc) { s.a[row][decltype(xc)::value] = part<C>(v[decltype(xc)::value]); });
+        __syncthreads();
+        if (active) static_for<0, NP>([&](auto yc) { part<C>(v[decltype(yc)::value]) = s.a[decltype(yc)::value][col]; });
+    });
+}
+
 }  // namespace tcx

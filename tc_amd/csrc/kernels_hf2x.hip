@@ -68,62 +68,6 @@ __global__ __launch_bounds__(256) void k_coulomb_table(T* __restrict__ table, co
     table[(long long)blockIdx.y * N + e] = static_cast<T>(g2 < 1e-8 ? 0.0 : invN / g2);
 }
 
-// LDS tile of one component (real or imaginary part) of a plane, [y][x] with one
-// element of padding per row.  The FP64 pass B transposes the two parts one after
-// the other: that halves its LDS per plane and doubles its waves per SIMD (1 -> 2 at
-// 40^3).  FP32 keeps whole complex tiles: split tiles would double its waves too
-// (2 -> 4), but with twice the LDS instructions and three times the barriers the
-// pass ran 5% slower.
-template <typename T, int NP>
-struct PartTile {
-    T a[NP][NP + 1];
-};
-template <int C, typename T>
-__device__ __forceinline__ T& part(cpx<T>& z)
-{
-    if constexpr (C == 0) return z.re; else return z.im;
-}
-
-// Transposes of the PL planes of a workgroup: thread t (active) holds column x=t
-// (values along y) -> row y=t (values along x), and back.  Every thread of the
-// workgroup calls them (they contain the barriers).
-template <typename T, int NP>
-__device__ __forceinline__ void cols_to_rows(PlaneTile<T, NP>& s, cpx<T> (&v)[NP], int t, bool active)
-{
-    if (active) tile_put_col<T, NP>(s, v, t);
-    __syncthreads();
-    if (active) tile_get_row<T, NP>(s, v, t);
-}
-template <typename T, int NP>
-__device__ __forceinline__ void rows_to_cols(PlaneTile<T, NP>& s, cpx<T> (&v)[NP], int t, bool active)
-{
-    if (active) tile_put_row<T, NP>(s, v, t);  // row t was read by thread t alone
-    __syncthreads();
-    if (active) tile_get_col<T, NP>(s, v, t);
-}
-template <typename T, int NP>
-__device__ __forceinline__ void cols_to_rows(PartTile<T, NP>& s, cpx<T> (&v)[NP], int t, bool active)
-{
-    static_for<0, 2>([&](auto cc) {
-        constexpr int C = decltype(cc)::value;
-        if constexpr (C == 1) __syncthreads();  // every thread has read the real parts
-        if (active) static_for<0, NP>([&](auto yc) { s.a[decltype(yc)::value][t] = part<C>(v[decltype(yc)::value]); });
-        __syncthreads();
-        if (active) static_for<0, NP>([&](auto xc) { part<C>(v[decltype(xc)::value]) = s.a[t][decltype(xc)::value]; });
-    });
-}
-template <typename T, int NP>
-__device__ __forceinline__ void rows_to_cols(PartTile<T, NP>& s, cpx<T> (&v)[NP], int t, bool active)
-{
-    static_for<0, 2>([&](auto cc) {
-        constexpr int C = decltype(cc)::value;
-        if constexpr (C == 1) __syncthreads();
-        if (active) static_for<0, NP>([&](auto xc) { s.a[t][decltype(xc)::value] = part<C>(v[decltype(xc)::value]); });
-        __syncthreads();
-        if (active) static_for<0, NP>([&](auto yc) { part<C>(v[decltype(yc)::value]) = s.a[decltype(yc)::value][t]; });
-    });
-}
-
 // One workgroup transforms PL planes of one pair (PlaneGroup): thread t owns
 // line t % NP of plane t / NP.  Column load (coalesced) -> FFT_y -> LDS
 // transpose -> FFT_x -> x v(G)/N -> inverse FFT_x -> LDS transpose -> inverse
@@ -134,7 +78,7 @@ __global__ __launch_bounds__((PlaneGroup<T, NP>::threads)) void k_hf2x_B(cpx<T>*
                                                                        const T* __restrict__ table, int kq0, int nz)
 {
     constexpr int PL = PlaneGroup<T, NP>::planes;
-    using Tile = std::conditional_t<sizeof(T) == 8, PartTile<T, NP>, PlaneTile<T, NP>>;
+    using Tile = TransposeTile<T, NP>;
     __shared__ Tile tiles[PL];
     const int p = threadIdx.x / NP, t = threadIdx.x % NP;
     const int z = blockIdx.x * PL + p;
@@ -147,7 +91,7 @@ __global__ __launch_bounds__((PlaneGroup<T, NP>::threads)) void k_hf2x_B(cpx<T>*
         load_pencil_nt<T, NP>(v, plane + t, NP);
         fft<T, NP, -1>(v);
     }
-    cols_to_rows<T, NP>(tile, v, t, active);
+    cols_to_rows<T, NP>(tile, v, t, t, active);
     if (active) {
         fft<T, NP, -1>(v);
         // frequency (x, y=t, z); the table is y-fastest within the plane
@@ -158,7 +102,7 @@ __global__ __launch_bounds__((PlaneGroup<T, NP>::threads)) void k_hf2x_B(cpx<T>*
         });
         fft<T, NP, 1>(v);
     }
-    rows_to_cols<T, NP>(tile, v, t, active);
+    rows_to_cols<T, NP>(tile, v, t, t, active);
     if (active) {
         fft<T, NP, 1>(v);
         store_pencil_nt<T, NP>(v, plane + t, NP);

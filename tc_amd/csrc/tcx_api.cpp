@@ -244,6 +244,7 @@ void Context::hermitian_conj()
 
 void Context::invalidate_states()
 {
+    if (!basis_set) cols.valid = false;
     clear_zero_weight();  // its states live in the orbital arrays that a setter replaces
     invalidate_local();
     occR_valid[0] = occR_valid[1] = false;
@@ -548,18 +549,40 @@ void Context::ensure_gradR(int prec)
 // Launch shape: every launch pairs a block of consecutive targets (k,j) with a
 // block of consecutive sources (q,i).  Targets own their accumulation grid
 // within a launch, so launches of one apply are serialised on the stream and
-// W needs no atomics.  Auto shape: enough targets that pass C issues
-// kAutoTargetWaves wavefronts, then as many sources as kAutoBufferGrids pair
-// grids allow (channels = grids per pair record: 1 for hf2x, 4 for tc2x).
-void Context::resolve_shape(int term, long& tc, long& sc, long ntargets, long nsources) const
+// W needs no atomics.  Auto shape, plane-first: sources whose planes on one XCD (an
+// eighth of them, see k_plane_A) fit its 4 MB L2 with room for the targets', a whole
+// number of pass C groups; targets for four rounds of pass C workgroups over the CUs; both
+// split evenly.  40^3 FP32, 1024 x 1024 orbitals: 94 x 48.  Per apply 96 sources take 20 ms
+// more (pass A reads beyond L2), 32 take 10 ms more and 64 targets 12 ms more (pass C:
+// fewer pairs per update of W; a part-filled last round).
+// Z-first: enough targets that pass C issues kAutoTargetWaves wavefronts, then as many
+// sources as kAutoBufferGrids pair grids allow (channels = grids per pair record: 1 for
+// hf2x, 4 for tc2x).
+void Context::resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources) const
 {
     constexpr long kAutoTargetWaves = 8192, kAutoBufferGrids = 8192;
+    constexpr long kXcds = 8, kL2Share = 3 << 20, kRounds = 4, kRecordBytes = (long)4 << 30;
     const int channels = term == 1 ? 4 : 1;
+    ntargets = std::max<long>(1, ntargets);
+    nsources = std::max<long>(1, nsources);
     const long waves_per_target = ((long)geo.n1 * geo.n2 + 31) / 32;
-    tc = shape_targets[term] > 0 ? shape_targets[term] : (kAutoTargetWaves + waves_per_target - 1) / waves_per_target;
-    tc = std::max<long>(1, std::min(tc, std::max<long>(1, ntargets)));
-    sc = shape_sources[term] > 0 ? shape_sources[term] : std::max<long>(1, kAutoBufferGrids / channels / tc);
-    sc = std::max<long>(1, std::min(sc, std::max<long>(1, nsources)));
+    tc = (kAutoTargetWaves + waves_per_target - 1) / waves_per_target;
+    sc = 0;
+    if (term == 0 && use_plane_first(prec)) {
+        const long grid_bytes = (long)N * 8;
+        const PlaneShape ps = plane_shape(geo.n1);
+        auto even = [](long n, long most) { return (n + (n + most - 1) / most - 1) / ((n + most - 1) / most); };
+        auto whole = [&](long n) { return std::max<long>(1, n / ps.group) * ps.group; };
+        const long most = whole(kXcds * kL2Share / grid_bytes);
+        sc = std::min(most, whole(even(nsources, most) + ps.group - 1));
+        tc = std::max<long>(1, kRounds * ps.slots / geo.n3);
+        tc = even(ntargets, std::max<long>(1, std::min(tc, kRecordBytes / (sc * grid_bytes))));
+    }
+    if (shape_targets[term] > 0) tc = shape_targets[term];
+    tc = std::max<long>(1, std::min(tc, ntargets));
+    if (sc == 0) sc = std::max<long>(1, kAutoBufferGrids / channels / tc);
+    if (shape_sources[term] > 0) sc = shape_sources[term];
+    sc = std::max<long>(1, std::min(sc, nsources));
     while (tc * sc > 65535) {
         if (sc > 1)
             sc = std::max<long>(1, 65535 / tc);
@@ -637,12 +660,13 @@ std::vector<PairItem> Context::occupied_items(bool irreducible_only) const
     return v;
 }
 
-const Plan& Context::get_plan(const std::vector<int>& nb, int term)
+// term 0: hf2x, 1: tc2x, kPlanJobs: the per-band jobs without the band pairs
+const Plan& Context::get_plan(const std::vector<int>& nb, int term, int prec)
 {
     long nt = 0;
     for (int k = 0; k < nk; ++k) nt += nb[k];
-    long tc, sc;
-    resolve_shape(term, tc, sc, nt, n_occ);
+    long tc = 0, sc = 0;
+    if (term != kPlanJobs) resolve_shape(term, prec, tc, sc, nt, n_occ);
     auto key = std::make_tuple(nb, tc, sc);
     auto it = plans.find(key);
     if (it != plans.end()) return it->second;
@@ -654,7 +678,9 @@ const Plan& Context::get_plan(const std::vector<int>& nb, int term)
         P.app_coef[k + 1] = P.app_coef[k] + (long long)nb[k] * npw[k];
     }
     P.n_app = (int)P.app_first[nk];
-    if (nspin == 1) {
+    if (term == kPlanJobs) {
+        // no pairs
+    } else if (nspin == 1) {
         build_pairs(P, applied_items(nb), occupied_items(), tc, sc, kcart, false);
     } else {
         // the exchange pairs states of one spin only (calc_hamiltonian_hf2x.cpp:46, :90-134)
@@ -785,7 +811,7 @@ void Context::hf2x(const int* nb_, const double* phi, double* out, int prec, uns
 {
     check_apply_args(nb_, phi, out, prec);
     std::vector<int> nb(nb_, nb_ + nk);
-    const Plan& P = get_plan(nb, 0);
+    const Plan& P = get_plan(nb, 0, prec);
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     if (P.n_app > 0) {
         ensure_occR(prec);

@@ -41,6 +41,14 @@ struct Geom {
     double b[9];   // reciprocal rows b_i: b[3*i + d]
 };
 
+// Support columns of the plane-first pair records (kernels_plane.hip): run[kx] = lo | len << 8 |
+// first << 16 over ky rotated by rot, colxy[c] = i1 | i2 << 16.
+struct PlaneCols {
+    const int* run;
+    const int* colxy;
+    int ncol, cstride, rot;
+};
+
 // One (k,j,q,i) pair of a launch: indices into the real-space grid arrays.
 struct PairEntry {
     int app;   // applied-orbital grid (k, j)
@@ -122,14 +130,21 @@ void launch_fft_xy(int prec, int sign, void* grids, int ngrids, const Geom& g, h
 void launch_fft_z(int prec, int sign, void* grids, int ngrids, const Geom& g, double scale, hipStream_t s);
 
 // hf2x pair pipeline
-// plane-first hf2x (kernels_hf2x_xy.hip), FP32-split
-void launch_hf2x_xyA(const Geom& g, const void* app, const void* occ, const PairEntry* pairs, int npairs,
-                     const int* colxy, const int* coloff, void* rec, int cstride, hipStream_t s);
-void launch_hf2x_zB(const Geom& g, void* rec, const PairEntry* pairs, int npairs, const int* colxy, const int* coloff,
-                    const double* kqcart, int cstride, hipStream_t s);
-void launch_hf2x_xyC(const Geom& g, const void* rec, const void* occ, const PairEntry* pairs,
-                     const TargetEntry* targets, int ntargets, const int* rowinfo, const double* fill, double* W,
-                     float* Wc, int cstride, hipStream_t s);
+// plane-first hf2x (kernels_plane.hip)
+// pairs that pass C sums at a time, and its workgroups that the GPU holds at once
+struct PlaneShape {
+    int group, slots;
+};
+PlaneShape plane_shape(int n1);
+void launch_plane_A(const Geom& g, const void* app, const void* occ, const PairEntry* pairs, int ntargets,
+                    int nsrc, const PlaneCols& pc, void* rec, hipStream_t s);
+void launch_plane_coulomb(void* tab, const double* kqcart, int row0, int nrows, const PlaneCols& pc,
+                          const Geom& g, hipStream_t s);
+void launch_plane_Z(const Geom& g, void* rec, const PairEntry* pairs, int npairs, const void* tab, int kq0,
+                    const PlaneCols& pc, hipStream_t s);
+void launch_plane_C(const Geom& g, const void* rec, const void* occ, const PairEntry* pairs,
+                    const TargetEntry* targets, int ntargets, const PlaneCols& pc, const double* fill, double* W,
+                    float* Wc, hipStream_t s);
 void launch_hf2x_A(int prec, const Geom& g, const void* phiR_app, const void* phiR_occ, const PairEntry* pairs,
                    int npairs, void* buf, hipStream_t s);
 void launch_coulomb_table(int prec, void* table, const double* kqcart, int row0, int nrows, const Geom& g,

@@ -99,7 +99,7 @@ void Context::tc3a3b3b4b6(const int* nb_, const double* phi, double* out, int pr
     require(method != TCX_METHOD_HF, TCX_ERR_STATE, "tc3a3b3b4b6: the cell was set up for HF");
     require(jastrow_set, TCX_ERR_STATE, "tc3a3b3b4b6: call tcx_set_jastrow_rpa first");
     std::vector<int> nb(nb_, nb_ + nk);
-    const Plan& P = get_plan(nb, 0);
+    const Plan& P = get_plan(nb, kPlanJobs);
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     // u = 0 makes every contribution vanish, and the G=0 correction is skipped with it (:99)
     if (P.n_app > 0 && n_occ > 0 && !u_zero()) {
@@ -408,7 +408,7 @@ void Context::tc3a2a4b2b5(const int* nb_, const double* phi, double* out, int pr
     require(method != TCX_METHOD_HF, TCX_ERR_STATE, "tc3a2a4b2b5: the cell was set up for HF");
     require(jastrow_set, TCX_ERR_STATE, "tc3a2a4b2b5: call tcx_set_jastrow_rpa first");
     std::vector<int> nb(nb_, nb_ + nk);
-    const Plan& P = get_plan(nb, 0);
+    const Plan& P = get_plan(nb, kPlanJobs);
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     if (P.n_app > 0 && n_occ > 0 && !u_zero()) {
         const bool bitc = method == TCX_METHOD_BITC;
@@ -529,7 +529,7 @@ void Context::kinetic(const int* nb_, const double* phi, double* out, unsigned f
     require(nb_ && phi && out, TCX_ERR_ARG, "kinetic: null pointer");
     for (int k = 0; k < nk; ++k) require(nb_[k] >= 0, TCX_ERR_ARG, "kinetic: negative band count");
     std::vector<int> nb(nb_, nb_ + nk);
-    const Plan& P = get_plan(nb, 0);
+    const Plan& P = get_plan(nb, kPlanJobs);
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     if (P.n_app > 0)
         launch_kinetic(io.phi, (const int*)d_gindex.p, (const OrbEntry*)P.d_appjobs.p, P.n_app, max_npw,
@@ -541,7 +541,7 @@ void Context::hf2h(const int* nb_, const double* phi, double* out, unsigned flag
 {
     check_apply_args(nb_, phi, out, TCX_PREC_FP64);
     std::vector<int> nb(nb_, nb_ + nk);
-    const Plan& P = get_plan(nb, 0);
+    const Plan& P = get_plan(nb, kPlanJobs);
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     if (P.n_app > 0 && n_occ > 0) {
         const size_t g = (size_t)N * 16;
@@ -566,7 +566,7 @@ void Context::tc2h(const int* nb_, const double* phi, double* out, unsigned flag
     require(method != TCX_METHOD_HF, TCX_ERR_STATE, "tc2h: the cell was set up for HF");
     require(jastrow_set, TCX_ERR_STATE, "tc2h: call tcx_set_jastrow_rpa first");
     std::vector<int> nb(nb_, nb_ + nk);
-    const Plan& P = get_plan(nb, 0);
+    const Plan& P = get_plan(nb, kPlanJobs);
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     if (P.n_app > 0 && n_occ > 0) {
         const bool bitc = method == TCX_METHOD_BITC;

@@ -80,22 +80,12 @@ struct PairItem {
 void build_pairs(PairSet& S, const std::vector<PairItem>& tg, const std::vector<PairItem>& src, long tc, long sc,
                  const std::vector<double>& kcart, bool same_k);
 
-// Support columns of the plane-first hf2x records, per k-q row of a pair set
-// (kernels_hf2x_xy.hip): colxy[coloff[r] + c] = i1 | i2 << 16, rowinfo[r][i2] = (lo, len).
-struct XyColumns {
-    bool built = false;
-    int cstride = 0;      // record columns per plane (the largest row)
-    double mean_cols = 0; // mean columns per pair
-    DBuf d_colxy, d_coloff, d_rowinfo;
-};
-
 struct Plan : PairSet {
     std::vector<long long> app_first, app_coef;  // per k: first applied orbital, coefficient offset
     int n_app = 0;
     DBuf d_appjobs;      // OrbEntry per applied band (band order)
     DBuf d_appgradjobs;  // three OrbEntry (dir 0..2) per applied band
     DBuf d_divjobs;      // DivEntry per applied band
-    mutable XyColumns xy;
 };
 
 // synchronous host -> device copy into a growing buffer
@@ -172,8 +162,15 @@ struct Context {
     long shape_sources[3] = {0, 0, 0};
     int hf2x_order = -1;          // -1 automatic, 0 z-first, 1 plane-first (FP32)
     double hf2x_record_cols = 0;  // (kx, ky) columns per plane of the last hf2x apply's records
+    bool in_davidson = false;     // an apply of tcx_davidson runs (use_plane_first)
     bool use_plane_first(int prec) const;
-    void build_xy_columns(const Plan& P);
+    // support columns of the pair records, from the basis (dropped by tcx_set_basis and what precedes it)
+    struct {
+        bool valid = false;
+        PlaneCols pc{};
+        DBuf buf;
+    } cols;
+    const PlaneCols& plane_cols();
     void hf2x_plane_first(const Plan& P);
     std::map<std::tuple<std::vector<int>, long, long>, Plan> plans;
     // pair sets of the three-body exchange terms, keyed by (applied bands, kind)
@@ -300,8 +297,9 @@ struct Context {
     void jastrow_kernels(int s1, int s2, long long n, const double* G2, double* uk, double* v);
     void ensure_density();
 
-    void resolve_shape(int term, long& tc, long& sc, long ntargets, long nsources) const;
-    const Plan& get_plan(const std::vector<int>& nb, int term);
+    void resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources) const;
+    static constexpr int kPlanJobs = -1;
+    const Plan& get_plan(const std::vector<int>& nb, int term, int prec = 0);
     void check_apply_args(const int* nb, const double* phi, const double* out, int prec);
     ApplyIO begin_apply(const int* nb, const double* phi, double* out, unsigned flags, const Plan& P);
     void end_apply(const ApplyIO& io);

@@ -76,3 +76,24 @@ def test_pipeline_order_errors(engine):
         with pytest.raises(tcx.TcxError) as e:
             engine.set_pipeline_order(term, order)
         assert e.value.code == tcx.TCX_ERR_ARG
+
+
+@pytest.mark.parametrize("gw,mesh", [(1.0, (4, 1, 1)), (1.35, (4, 3, 1)), (2.2, (2, 2, 1))])
+def test_plane_first_wrapping_columns(engine, gw, mesh):
+    """Bases whose differences reach past the grid (gw: multiple of the alias-free radius): the
+    runs of the column set that wrap take every ky, and the two orders stay equal to FP32
+    rounding and the oracle within the FP32-split bound."""
+    lat = S.fcc_lattice(6.0)
+    sys_ = S.build_system(lat, (18, 18, 12), mesh, nbands=3, nocc=2, seed_stream=530,
+                          gw=gw * S.gw_rule(lat, (18, 18, 12)))
+    engine.load_system(sys_)
+    nb = np.full(sys_.nk, 2, np.int32)
+    _, phi = S.applied_bands(sys_, nb=nb, seed=531)
+    ref = O.Oracle(sys_).hf2x(nb, phi)
+    out = {}
+    for order in (1, 0):
+        engine.set_pipeline_order("hf2x", order)
+        out[order] = engine.hf2x(nb, phi, precision=tcx.PREC_FP32)
+        assert per_band_rel(sys_, nb, out[order], ref).max() <= 3e-5
+    engine.set_pipeline_order("hf2x", -1)
+    assert per_band_rel(sys_, nb, out[1], out[0]).max() <= 1e-6
