@@ -36,15 +36,17 @@ using PT = float;  // precision of the pair records
 
 // Workgroup of the plane passes: R tiles (planes of a pair in pass A, pairs of a plane in
 // pass C) of NP lines each, line t of tile r on thread r NP + t.  R fills the wavefronts best
-// among those that leave 8 wavefronts (2 per SIMD) of workgroups in a CU's 160 KB of LDS.
+// among those that leave 8 wavefronts (2 per SIMD) of workgroups in a CU's 160 KB of LDS, with
+// at most 16 accumulators a thread (a single 48-line tile would hold 48 of them: 48^3 ran at two
+// thirds of the z-first speed).
 template <typename T, int NP>
 struct PlaneWg {
     static constexpr int tile_bytes = (int)sizeof(PlaneTile<T, NP>);
     static constexpr int pick()
     {
-        int best = 1;
+        int best = (NP + 15) / 16;
         double best_score = 0.0;
-        for (int r = 1; r <= 16 && r * NP <= 256 && r * tile_bytes <= 80 * 1024; ++r) {
+        for (int r = (NP + 15) / 16; r <= 16 && r * NP <= 256 && r * tile_bytes <= 80 * 1024; ++r) {
             const int waves = (r * NP + 63) / 64;
             const int per_cu = (160 * 1024) / (r * tile_bytes) * waves;
             const double score = double(r * NP) / (64 * waves) * (per_cu >= 8 ? 1.0 : per_cu / 8.0);
@@ -115,7 +117,7 @@ __device__ __forceinline__ void load_row(cpx<T> (&v)[NP], const cpx<T>* plane, c
 // Plane-group-fastest order also keeps the record writes in flight close together: a
 // plane-slowest order, which gives each XCD a fixed set of planes too, took 139 ms.
 template <typename T, int NP>
-__global__ __launch_bounds__((PlaneWg<T, NP>::threads)) void k_plane_A(const cpx<T>* __restrict__ phiR_app,
+__global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_A(const cpx<T>* __restrict__ phiR_app,
                                                                      const cpx<T>* __restrict__ phiR_occ,
                                                                      const PairEntry* __restrict__ pairs, int nsrc,
                                                                      const int* __restrict__ runs, PlaneCols pc,
@@ -177,7 +179,7 @@ __global__ __launch_bounds__(256) void k_plane_coulomb(T* __restrict__ tab, cons
 
 // Pass Z: one lane per support column of a pair, its whole z pencil in registers.
 template <typename T, int NZ>
-__global__ __launch_bounds__(kPencilBlock) void k_plane_Z(cpx<T>* __restrict__ rec, const PairEntry* __restrict__ pairs,
+__global__ __launch_bounds__(kPencilBlock, 2) void k_plane_Z(cpx<T>* __restrict__ rec, const PairEntry* __restrict__ pairs,
                                                           const T* __restrict__ tab, int kq0, PlaneCols pc)
 {
     const int c = blockIdx.x * kPencilBlock + threadIdx.x;
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(kPencilBlock) void k_plane_Z(cpx<T>* __restrict__ r
 // 40^3) with whole lines per lane: split lines (4 lanes each, the accumulators by line) cost
 // twice the instructions and ran 2.7 times longer.
 template <typename T, int NP>
-__global__ __launch_bounds__((PlaneWg<T, NP>::threads)) void k_plane_C(
+__global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_C(
     const cpx<T>* __restrict__ rec, const cpx<T>* __restrict__ phiR_occ, const PairEntry* __restrict__ pairs,
     const TargetEntry* __restrict__ targets, const int* __restrict__ runs, PlaneCols pc,
     const double* __restrict__ fill, cpx<double>* __restrict__ W, float2* __restrict__ Wc, int nz)
