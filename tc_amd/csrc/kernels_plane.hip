@@ -25,88 +25,14 @@
 // that every index below is uniform over a launch.  kx by kx, a contiguous run of rotated
 // ky (t = (i2 - rot) mod n2), run[kx] = lo | len << 8 | first << 16; record [z][c].  A lane
 // owns one row t, so the lanes of a load or store of one kx are consecutive columns.
-#include "kernels_common.hpp"
+#include "plane_dev.hpp"
 #include "size_switch.hpp"
 
 namespace tcx {
 
 namespace {
-
 using PT = float;  // precision of the pair records
-
-// Workgroup of the plane passes: R tiles (planes of a pair in pass A, pairs of a plane in
-// pass C) of NP lines each, line t of tile r on thread r NP + t.  R fills the wavefronts best
-// among those that leave 8 wavefronts (2 per SIMD) of workgroups in a CU's 160 KB of LDS, with
-// at most 16 accumulators a thread (a single 48-line tile would hold 48 of them: 48^3 ran at two
-// thirds of the z-first speed).
-template <typename T, int NP>
-struct PlaneWg {
-    static constexpr int tile_bytes = (int)sizeof(PlaneTile<T, NP>);
-    static constexpr int pick()
-    {
-        int best = (NP + 15) / 16;
-        double best_score = 0.0;
-        for (int r = (NP + 15) / 16; r <= 16 && r * NP <= 256 && r * tile_bytes <= 80 * 1024; ++r) {
-            const int waves = (r * NP + 63) / 64;
-            const int per_cu = (160 * 1024) / (r * tile_bytes) * waves;
-            const double score = double(r * NP) / (64 * waves) * (per_cu >= 8 ? 1.0 : per_cu / 8.0);
-            if (score > best_score + 1e-9) {
-                best_score = score;
-                best = r;
-            }
-        }
-        return best;
-    }
-    static constexpr int R = pick();
-    static constexpr int threads = ((R * NP + 63) / 64) * 64;
-    static constexpr int rows = (NP + R - 1) / R;  // plane rows a thread sums in pass C
-};
-
-// The runs of a column set, read once per workgroup into scalar registers.
-template <int NP>
-struct PlaneRuns {
-    int run[NP];
-    __device__ __forceinline__ explicit PlaneRuns(const int* __restrict__ p)
-    {
-        static_for<0, NP>([&](auto xc) { run[decltype(xc)::value] = p[decltype(xc)::value]; });
-    }
-    // column (kx = x, row t) is kept, at base(x) + t
-    __device__ __forceinline__ bool has(int x, int t) const
-    {
-        return (unsigned)(t - (run[x] & 0xff)) < (unsigned)((run[x] >> 8) & 0xff);
-    }
-    __device__ __forceinline__ int base(int x) const { return (run[x] >> 16) - (run[x] & 0xff); }
-};
-
-template <typename T>
-__device__ __forceinline__ void store_nt(cpx<T>* p, cpx<T> x)
-{
-    typedef T v2 __attribute__((ext_vector_type(2)));
-    const v2 s = {x.re, x.im};
-    __builtin_nontemporal_store(s, reinterpret_cast<v2*>(p));
 }
-template <typename T>
-__device__ __forceinline__ cpx<T> load_nt(const cpx<T>* p)
-{
-    typedef T v2 __attribute__((ext_vector_type(2)));
-    const v2 x = __builtin_nontemporal_load(reinterpret_cast<const v2*>(p));
-    return cpx<T>{x.x, x.y};
-}
-// Row t of a record plane, zero outside the support.  The runs are read from memory at every
-// call (the empty asm hides that they do not change): held across a loop they would spill.
-template <typename T, int NP>
-__device__ __forceinline__ void load_row(cpx<T> (&v)[NP], const cpx<T>* plane, const int* __restrict__ runs, int t)
-{
-    asm volatile("" : "+s"(runs));
-    const PlaneRuns<NP> rr(runs);
-    static_for<0, NP>([&](auto xc) {
-        constexpr int x = decltype(xc)::value;
-        v[x] = cpx<T>{T(0), T(0)};
-        if (rr.has(x, t)) v[x] = load_nt(plane + t + rr.base(x));
-    });
-}
-
-}  // namespace
 
 // Pass A: R planes of one pair; pair = target tg x source s, nsrc sources per target.  Column
 // x = t of rho -> FFT_y -> LDS transpose -> row ky -> FFT_x -> the row's support columns.
@@ -134,27 +60,24 @@ __global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_A(const 
     const bool active = r < Wg::R && z < nz;
     int row = t + pc.rot;
     row = row >= NP ? row - NP : row;
-    const PlaneRuns<NP> runs_(runs);
     const PairEntry pe = pairs[p];
-    const size_t ng = (size_t)NP * NP * nz, o = (size_t)z * (NP * NP) + t;
+    const size_t ng = (size_t)NP * NP * nz, o = (size_t)grp * Wg::R * (NP * NP);
     cpx<T> v[NP];
     if (active) {
         const cpx<T>* a = phiR_app + (size_t)pe.app * ng + o;
         const cpx<T>* b = phiR_occ + (size_t)pe.occ * ng + o;
+        const unsigned off = (unsigned)(r * (NP * NP) + t) * sizeof(cpx<T>);
         static_for<0, NP>([&](auto yc) {
             constexpr int y = decltype(yc)::value;
-            v[y] = cmulc(b[y * NP], a[y * NP]);
+            v[y] = cmulc(ld<cpx<T>>(b + y * NP, off), ld<cpx<T>>(a + y * NP, off));
         });
         fft<T, NP, -1>(v);
     }
     cols_to_rows<T, NP>(tiles[active ? r : 0], v, t, row, active);
     if (active) {
         fft<T, NP, -1>(v);
-        cpx<T>* out = rec + ((size_t)p * nz + z) * pc.cstride + t;
-        static_for<0, NP>([&](auto xc) {
-            constexpr int x = decltype(xc)::value;
-            if (runs_.has(x, t)) store_nt(out + runs_.base(x), v[x]);
-        });
+        store_row<T, NP>(v, rec + ((size_t)p * nz + grp * Wg::R) * pc.cstride,
+                         (unsigned)(r * pc.cstride + t) * sizeof(cpx<T>), runs, t);
     }
 }
 
@@ -184,17 +107,18 @@ __global__ __launch_bounds__(kPencilBlock, 2) void k_plane_Z(cpx<T>* __restrict_
 {
     const int c = blockIdx.x * kPencilBlock + threadIdx.x;
     if (c >= pc.ncol) return;
-    cpx<T>* col = rec + (size_t)blockIdx.y * NZ * pc.cstride + c;
-    const T* v = tab + (size_t)(pairs[blockIdx.y].kq - kq0) * NZ * pc.cstride + c;
+    cpx<T>* col = rec + (size_t)blockIdx.y * NZ * pc.cstride;
+    const T* v = tab + (size_t)(pairs[blockIdx.y].kq - kq0) * NZ * pc.cstride;
+    const unsigned off = (unsigned)c * sizeof(cpx<T>), voff = (unsigned)c * sizeof(T);
     cpx<T> x[NZ];
-    load_pencil_nt<T, NZ>(x, col, pc.cstride);
+    ld_column<T, NZ>(x, col, off, pc.cstride);
     fft<T, NZ, -1>(x);
     static_for<0, NZ>([&](auto zc) {
         constexpr int z = decltype(zc)::value;
-        x[z] = scale(x[z], v[(size_t)z * pc.cstride]);
+        x[z] = scale(x[z], ld<T>(v + (size_t)z * pc.cstride, voff));
     });
     fft<T, NZ, 1>(x);
-    store_pencil_nt<T, NZ>(x, col, pc.cstride);
+    st_column<T, NZ>(x, col, off, pc.cstride);
 }
 
 // Pass C: plane z of one target, R pairs at a time, pair r in tile r.  Row ky = t from the
@@ -222,11 +146,12 @@ __global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_C(
     cpx<double> acc[ROWS];  // points x = t, y = r + i R
     static_for<0, ROWS>([&](auto ic) { acc[decltype(ic)::value] = cpx<double>{0.0, 0.0}; });
     const int pend = te.pair0 + te.npair;
-    auto plane_of = [&](int pp) { return rec + ((size_t)pp * nz + z) * pc.cstride; };
+    auto plane_of = [&](int pp) { return rec + ((size_t)pp * nz + z) * pc.cstride; };  // uniform
+    const unsigned off = (unsigned)(r * nz * pc.cstride + t) * sizeof(cpx<T>);           // pair r of the group
     // the rows of the next group are loaded while the points of this one are summed (152 -> 147 ms
     // per apply at 40^3)
     cpx<T> v[NP];
-    if (r < R && te.pair0 + r < pend) load_row<T, NP>(v, plane_of(te.pair0 + r), runs, t);
+    if (r < R && te.pair0 + r < pend) load_row<T, NP>(v, plane_of(te.pair0), off, runs, t);
 #pragma unroll 1
     for (int p0 = te.pair0; p0 < pend; p0 += R) {
         const bool on = r < R && p0 + r < pend, next = r < R && p0 + R + r < pend;
@@ -242,7 +167,7 @@ __global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_C(
         }
         const int nr = pend - p0 < R ? pend - p0 : R;
         if (on) tile_put_col<T, NP>(tile, v, t);  // column t was read by this thread alone
-        if (next) load_row<T, NP>(v, plane_of(p0 + R + r), runs, t);
+        if (next) load_row<T, NP>(v, plane_of(p0 + R), off, runs, t);
         __syncthreads();
         if (r < R)
             for (int s = 0; s < nr; ++s) {
@@ -264,7 +189,7 @@ __global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_C(
         constexpr int i = decltype(ic)::value;
         if (i * R + R <= NP || i * R + r < NP) {
             const size_t e = o + (size_t)(i * R + r) * NP;
-            add_partial((double2*)(W + e), Wc + e, acc[i].re, acc[i].im);
+            add_partial((double2*)(W + e), Wc ? Wc + e : nullptr, acc[i].re, acc[i].im);
         }
     });
 }

@@ -85,6 +85,7 @@ struct Plan : PairSet {
     int n_app = 0;
     DBuf d_appjobs;      // OrbEntry per applied band (band order)
     DBuf d_appgradjobs;  // three OrbEntry (dir 0..2) per applied band
+    DBuf d_app2jobs;     // two OrbEntry (phi, |k+G|^2 phi) per applied band
     DBuf d_divjobs;      // DivEntry per applied band
 };
 
@@ -166,12 +167,21 @@ struct Context {
     bool use_plane_first(int prec) const;
     // support columns of the pair records, from the basis (dropped by tcx_set_basis and what precedes it)
     struct {
-        bool valid = false;
+        bool valid = false, no_alias = false;
         PlaneCols pc{};
         DBuf buf;
     } cols;
     const PlaneCols& plane_cols();
     void hf2x_plane_first(const Plan& P);
+    // the two-channel form of tc2x (kernels_plane_tc2x.hip) and its orbital sets per precision
+    bool tc2x_two_channel();
+    void ensure_tc2x_sets(int prec);
+    void orbital_sets(const double* coef, const OrbEntry* d_jobs, int norb, int nc, int prec, void* out);
+    void tc2x_plane_first(const Plan& P);
+    void tc2x_two_channel_z(const Plan& P);
+    DBuf d_bra[2], d_ket[2], a_bra[2], a_ket[2];  // a_: of the other orientation (hermitian_conj)
+    bool sets_valid[2] = {false, false}, a_sets_valid[2] = {false, false};
+    DBuf d_occ2jobs, d_occ5jobs;  // OrbEntry (phi, L) and (phi, L, g_d) per occupied orbital
     std::map<std::tuple<std::vector<int>, long, long>, Plan> plans;
     // pair sets of the three-body exchange terms, keyed by (applied bands, kind)
     std::map<std::tuple<std::vector<int>, int>, PairSet> pairsets;
@@ -297,7 +307,7 @@ struct Context {
     void jastrow_kernels(int s1, int s2, long long n, const double* G2, double* uk, double* v);
     void ensure_density();
 
-    void resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources) const;
+    void resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources);
     static constexpr int kPlanJobs = -1;
     const Plan& get_plan(const std::vector<int>& nb, int term, int prec = 0);
     void check_apply_args(const int* nb, const double* phi, const double* out, int prec);
