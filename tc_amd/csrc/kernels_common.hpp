@@ -65,6 +65,47 @@ __device__ __forceinline__ void add_partial(double2* w, float2* wc, double are, 
 }
 
 
+// Grid and record accesses as (uniform base) + (32-bit lane offset in bytes): the base stays in
+// scalar registers and every element of a line takes scalar arithmetic only.  With a per-lane
+// pointer each of a line's 40 accesses needs a 64-bit vector address of its own: an
+// instruction and two registers each (k_plane_Z at 40^3 took 226 registers, now 126).
+template <typename X>
+__device__ __forceinline__ X ld(const void* base, unsigned off)
+{
+    return *reinterpret_cast<const X*>((const char*)base + off);
+}
+template <typename T>
+__device__ __forceinline__ cpx<T> ld_nt(const void* base, unsigned off)
+{
+    typedef T v2 __attribute__((ext_vector_type(2)));
+    const v2 x = __builtin_nontemporal_load(reinterpret_cast<const v2*>((const char*)base + off));
+    return cpx<T>{x.x, x.y};
+}
+template <typename T>
+__device__ __forceinline__ void st_nt(void* base, unsigned off, cpx<T> x)
+{
+    typedef T v2 __attribute__((ext_vector_type(2)));
+    const v2 s = {x.re, x.im};
+    __builtin_nontemporal_store(s, reinterpret_cast<v2*>((char*)base + off));
+}
+// pencils of stride `stride` elements; streaming (non-temporal) variants as below
+template <typename T, int M>
+__device__ __forceinline__ void ld_pencil(cpx<T> (&v)[M], const cpx<T>* base, unsigned off, int stride)
+{
+    static_for<0, M>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        v[m] = ld<cpx<T>>(base + (size_t)m * stride, off);
+    });
+}
+template <typename T, int M>
+__device__ __forceinline__ void st_pencil_nt(const cpx<T> (&v)[M], cpx<T>* base, unsigned off, int stride)
+{
+    static_for<0, M>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        st_nt<T>(base + (size_t)m * stride, off, v[m]);
+    });
+}
+
 template <typename T, int NZ>
 __device__ __forceinline__ void load_pencil(cpx<T> (&v)[NZ], const cpx<T>* __restrict__ p, int stride)
 {

@@ -35,15 +35,16 @@ __global__ __launch_bounds__(kPencilBlock) void k_hf2x_A(const cpx<T>* __restric
     if (xy >= nxy) return;
     const PairEntry pe = pairs[blockIdx.y];
     const size_t ng = (size_t)nxy * NZ;
-    const cpx<T>* a = phiR_app + (size_t)pe.app * ng + xy;
-    const cpx<T>* b = phiR_occ + (size_t)pe.occ * ng + xy;
+    const cpx<T>* a = phiR_app + (size_t)pe.app * ng;
+    const cpx<T>* b = phiR_occ + (size_t)pe.occ * ng;
+    const unsigned off = (unsigned)xy * sizeof(cpx<T>);
     cpx<T> v[NZ];
     static_for<0, NZ>([&](auto zc) {
         constexpr int z = decltype(zc)::value;
-        v[z] = cmulc(b[(size_t)z * nxy], a[(size_t)z * nxy]);
+        v[z] = cmulc(ld<cpx<T>>(b + (size_t)z * nxy, off), ld<cpx<T>>(a + (size_t)z * nxy, off));
     });
     fft<T, NZ, -1>(v);
-    store_pencil_nt<T, NZ>(v, buf + (size_t)blockIdx.y * ng + xy, nxy);
+    st_pencil_nt<T, NZ>(v, buf + (size_t)blockIdx.y * ng, off, nxy);
 }
 
 // Coulomb kernel table of a launch: v(G)/N = 1/(N |k-q+G|^2), 0 below 1e-8
@@ -134,25 +135,26 @@ __global__ __launch_bounds__(kPencilBlock) void k_hf2x_C(const cpx<T>* __restric
     static_for<0, M>([&](auto kc) { acc[decltype(kc)::value] = cpx<double>{0.0, 0.0}; });
     // the pencil of pair pp + 1 is loaded before pair pp is transformed (FP32)
     constexpr bool kPrefetch = sizeof(T) == 4 && M <= 20;  // 48^3 pencils would drop to one wave
-    auto grid_of = [&](int pp) { return buf + (size_t)pp * ng + xy + (size_t)h * nxy; };
+    auto grid_of = [&](int pp) { return buf + (size_t)pp * ng; };
+    const unsigned ioff = (unsigned)(xy + h * nxy) * sizeof(cpx<T>), ooff = (unsigned)(xy + ob * M * nxy) * sizeof(cpx<T>);
     cpx<T> vn[M];
-    if (kPrefetch && te.npair > 0) load_pencil<T, M>(vn, grid_of(te.pair0), S * nxy);
+    if (kPrefetch && te.npair > 0) ld_pencil<T, M>(vn, grid_of(te.pair0), ioff, S * nxy);
 #pragma unroll 1
     for (int pp = te.pair0; pp < te.pair0 + te.npair; ++pp) {
         const int occ = pairs[pp].occ;
         cpx<T> v[M];
         if (kPrefetch) {
             static_for<0, M>([&](auto mc) { v[decltype(mc)::value] = vn[decltype(mc)::value]; });
-            if (pp + 1 < te.pair0 + te.npair) load_pencil<T, M>(vn, grid_of(pp + 1), S * nxy);
+            if (pp + 1 < te.pair0 + te.npair) ld_pencil<T, M>(vn, grid_of(pp + 1), ioff, S * nxy);
         } else {
-            load_pencil<T, M>(v, grid_of(pp), S * nxy);  // z = S m + h
+            ld_pencil<T, M>(v, grid_of(pp), ioff, S * nxy);  // z = S m + h
         }
         Split::template fft<T, NZ, 1, kSwapF64<T>>(v, h);  // -> z = ob*M + k
-        const cpx<T>* q = phiR_occ + (size_t)occ * ng + xy + (size_t)ob * M * nxy;
+        const cpx<T>* q = phiR_occ + (size_t)occ * ng;
         const double f = fill ? fill[occ] : 1.0;
         static_for<0, M>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
-            const cpx<T> prod = v[k] * q[(size_t)k * nxy];
+            const cpx<T> prod = v[k] * ld<cpx<T>>(q + (size_t)k * nxy, ooff);
             acc[k].re += f * static_cast<double>(prod.re);
             acc[k].im += f * static_cast<double>(prod.im);
         });

@@ -202,6 +202,20 @@ void launch_a3_b34(int prec, double* W, const double* qsum, const double* dnu, c
     });
 }
 
+__global__ __launch_bounds__(256) void k_sum3(double2* __restrict__ a, long long n)
+{
+    const long long r = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (r >= n) return;
+    a[r] = dadd(a[r], dadd(a[r + n], a[r + 2 * n]));
+}
+
+void launch_sum3(double* a, long long n, hipStream_t s)
+{
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_sum3, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (double2*)a, n);
+    TCX_HIP_CHECK(hipGetLastError());
+}
+
 // [3b6] divergence correction (tc3a3b3b4b6.cpp:424-451):
 //   tG(G) = sum_js 4 pi n_js(G) A_js u(G, 0, js) (G != 0),  tG(0) = 0
 template <bool kPoly>

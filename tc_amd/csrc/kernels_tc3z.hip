@@ -50,14 +50,6 @@ struct LaneOf {
     }
 };
 
-// v = FFT_backward along z of the pencil of grid g (split layout in, blocked layout out)
-template <typename T, int NZ, int S>
-__device__ __forceinline__ void zinv(cpx<T> (&v)[NZ / S], const cpx<T>* grid, const LaneOf<S>& L, int nxy)
-{
-    load_pencil<T, NZ / S>(v, grid + L.xy + (size_t)L.h * nxy, S * nxy);  // z = S m + h
-    PencilSplit<S>::template fft<T, NZ, 1>(v, L.h);                      // -> z = ob M + k
-}
-
 }  // namespace
 
 // ----------------------------------------------------------------- tc3a3b3b4b6 real-space step
@@ -157,142 +149,106 @@ __global__ __launch_bounds__(kPencilBlock) void k_za7_mid(cpx<T>* __restrict__ P
 }
 
 // ----------------------------------------------------------------- tc3a2a4b2b5 q-sums
-// Per target (q2,i2) over pairs (q1,i1), O[p][6h + 3s + d] (h = 1 only for BITC):
-//   Q2 -= f1 sum_{s,d} O_0,s,d conj(O_h2,s,d)     (h2 = 1 for BITC, 0 for TC)
-template <typename T, int NZ, int S>
-__global__ __launch_bounds__(kPencilBlock) void k_za8_q2(const cpx<T>* __restrict__ O, int bitc,
-                                                         const PairEntry* __restrict__ pairs,
-                                                         const TargetEntry* __restrict__ targets,
-                                                         const double* __restrict__ fill, double2* __restrict__ Q2,
-                                                         int nxy)
+// Per target t (q2,i2) and direction d = blockIdx.z, over its entries e = {record app, source
+// occ (q1,i1), role kq}; v = O_0,s,d and w = O_1,s,d of the record (O[rec][6h + 3s + d], h = 1 only
+// for BITC, else w = v):
+//   Q2[d] -= f1 sum_s v conj(w)
+//   Q4[d] += f1 v_0 phi_q1,   Q5[d] -= f1 conj(w_0 chi_q1)   (s = 0; Q5 for BITC only)
+// Role 1: the record is that of the reversed pair (target q1, source q2).  With K odd under the
+// exchange and rho_21 = conj of the other side's rho_12, O_0 of (q1, q2) is -conj(O_1) of
+// (q2, q1) and the reverse, so v and w change places, conjugated and negated, and v conj(w)
+// stays.  One pass reads each channel once and feeds all three sums (before, Q2 and Q4/Q5 read
+// and transformed 18 channels per pair in separate passes, now 12).
+// 40^3 FP32 BITC, 96 orbitals: 2.30 -> 1.67 us per ordered pair (3.7 TB/s of record reads; the
+// FP64 accumulators leave two waves per SIMD).
+// Two waves per SIMD where the accumulators leave room (the compiler took one for 36 points).
+template <typename T, int NZ, int S, bool kBitc>
+__global__ __launch_bounds__(kPencilBlock, (NZ / S <= (sizeof(T) == 4 ? 12 : 10) ? 2 : 1)) void k_za8_q(const cpx<T>* __restrict__ O, const cpx<T>* __restrict__ occR,
+                                                        const cpx<T>* __restrict__ chiR,
+                                                        const PairEntry* __restrict__ entries,
+                                                        const TargetEntry* __restrict__ targets,
+                                                        const double* __restrict__ fill, double2* __restrict__ Q2,
+                                                        size_t q2_slice, double2* __restrict__ Q4,
+                                                        double2* __restrict__ Q5, int nxy)
 {
     constexpr int M = NZ / S;
-    const LaneOf<S> L(nxy);
-    const TargetEntry te = targets[blockIdx.y];
-    const size_t ng = (size_t)nxy * NZ;
-    const int nch = bitc ? 12 : 6;
-    double2 acc[M];
-    static_for<0, M>([&](auto kc) { acc[decltype(kc)::value] = make_double2(0.0, 0.0); });
-    // steps it = 6 (pair) + c; the pencil(s) of step it + 1 are loaded before step it is
-    // transformed
-    const int nsteps = 6 * te.npair;
-    auto grid_of = [&](int it, int half) {
-        return O + ((size_t)(te.pair0 + it / 6) * nch + 6 * half + it % 6) * ng + L.xy + (size_t)L.h * nxy;
-    };
-    constexpr bool kPrefetch = sizeof(T) == 4;  // FP64 instances have no VGPRs to spare
-    cpx<T> vn[M], wn[M];
-    if (kPrefetch && nsteps > 0) {
-        load_pencil<T, M>(vn, grid_of(0, 0), S * nxy);  // z = S m + h
-        if (bitc) load_pencil<T, M>(wn, grid_of(0, 1), S * nxy);
-    }
-#pragma unroll 1
-    for (int it = 0; it < nsteps; ++it) {
-        const double f1 = fill[pairs[te.pair0 + it / 6].occ];
-        {
-            cpx<T> v[M];
-            if (kPrefetch) {
-                static_for<0, M>([&](auto mc) { v[decltype(mc)::value] = vn[decltype(mc)::value]; });
-                if (it + 1 < nsteps) load_pencil<T, M>(vn, grid_of(it + 1, 0), S * nxy);
-            } else {
-                load_pencil<T, M>(v, grid_of(it, 0), S * nxy);
-            }
-            PencilSplit<S>::template fft<T, NZ, 1>(v, L.h);  // -> z = ob M + k
-            if (bitc) {
-                cpx<T> w[M];
-                if (kPrefetch) {
-                    static_for<0, M>([&](auto mc) { w[decltype(mc)::value] = wn[decltype(mc)::value]; });
-                    if (it + 1 < nsteps) load_pencil<T, M>(wn, grid_of(it + 1, 1), S * nxy);
-                } else {
-                    load_pencil<T, M>(w, grid_of(it, 1), S * nxy);
-                }
-                PencilSplit<S>::template fft<T, NZ, 1>(w, L.h);
-                static_for<0, M>([&](auto kc) {
-                    constexpr int k = decltype(kc)::value;
-                    const double2 a = upd(v[k]), b = upd(w[k]);
-                    acc[k] = cmadd(acc[k], a, make_double2(b.x, -b.y), -f1);
-                });
-            } else {
-                static_for<0, M>([&](auto kc) {
-                    constexpr int k = decltype(kc)::value;
-                    const double2 a = upd(v[k]);
-                    acc[k].x -= f1 * (a.x * a.x + a.y * a.y);
-                });
-            }
-        }
-    }
-    if (!L.valid) return;
-    double2* q = Q2 + (size_t)te.app * ng + L.xy + (size_t)L.ob * M * nxy;
-    static_for<0, M>([&](auto kc) {
-        constexpr int k = decltype(kc)::value;
-        const double2 a = q[(size_t)k * nxy];
-        q[(size_t)k * nxy] = make_double2(a.x + acc[k].x, a.y + acc[k].y);
-    });
-}
-
-// Q4[d] += f1 O_0,0,d phi_q1     (conj5 = 0, channel d, X = occupied right orbitals)
-// Q5[d] -= f1 conj(O_1,0,d chi_q1)  (conj5 = 1, channel 6 + d, X = occupied left orbitals; BITC)
-// with d = blockIdx.z.
-template <typename T, int NZ, int S>
-__global__ __launch_bounds__(kPencilBlock) void k_za8_q45(const cpx<T>* __restrict__ O, int nch, int ch0, int conj5,
-                                                          const cpx<T>* __restrict__ X,
-                                                          const PairEntry* __restrict__ pairs,
-                                                          const TargetEntry* __restrict__ targets,
-                                                          const double* __restrict__ fill, double2* __restrict__ Q,
-                                                          int nxy)
-{
-    constexpr int M = NZ / S;
+    constexpr int nch = kBitc ? 12 : 6;
     const LaneOf<S> L(nxy);
     const TargetEntry te = targets[blockIdx.y];
     const int d = blockIdx.z;
     const size_t ng = (size_t)nxy * NZ;
     const size_t o0 = L.xy + (size_t)L.ob * M * nxy;
-    const double sy = conj5 ? -1.0 : 1.0;  // conj flips the imaginary part; Q5 also flips the sign
-    double2 acc[M];
-    static_for<0, M>([&](auto kc) { acc[decltype(kc)::value] = make_double2(0.0, 0.0); });
-    // the pencil of pair pp + 1 is loaded before pair pp is transformed (FP32)
-    constexpr bool kPrefetch = sizeof(T) == 4;
-    auto grid_of = [&](int pp) { return O + ((size_t)pp * nch + ch0 + d) * ng + L.xy + (size_t)L.h * nxy; };
+    double2 q2[M], q4[M], q5[kBitc ? M : 1];
+    static_for<0, M>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        q2[k] = make_double2(0.0, 0.0);
+        q4[k] = make_double2(0.0, 0.0);
+        if constexpr (kBitc) q5[k] = make_double2(0.0, 0.0);
+    });
+    // FP32 up to 40^3: the h = 0 pencil of the next (entry, s) step is loaded before this one is
+    // transformed, the h = 1 pencil when v's registers are its own: 15.4 ms against 17.4 without
+    // (96 orbitals at 40^3); both pencils ahead would spill
+    constexpr bool kPrefetch = sizeof(T) == 4 && M <= 10;
+    auto chan = [&](int rec, int h, int s) { return O + ((size_t)rec * nch + 6 * h + 3 * s + d) * ng; };
+    const unsigned ioff = (unsigned)(L.xy + L.h * nxy) * sizeof(cpx<T>), ooff = (unsigned)o0 * sizeof(cpx<T>);
     cpx<T> vn[M];
-    if (kPrefetch && te.npair > 0) load_pencil<T, M>(vn, grid_of(te.pair0), S * nxy);
+    auto load = [&](int rec, int s) { ld_pencil<T, M>(vn, chan(rec, 0, s), ioff, S * nxy); };  // z = S m + h
+    const int end = te.pair0 + te.npair;
+    if (kPrefetch && te.npair > 0) load(entries[te.pair0].app, 1);
 #pragma unroll 1
-    for (int pp = te.pair0; pp < te.pair0 + te.npair; ++pp) {
-        const PairEntry e = pairs[pp];
+    for (int i = te.pair0; i < end; ++i) {
+        const PairEntry e = entries[i];
         const double f1 = fill[e.occ];
-        const cpx<T>* xg = X + (size_t)e.occ * ng + o0;
-        cpx<T> v[M];
-        if (kPrefetch) {
+        const bool rev = e.kq != 0;
+        static_for<0, 2>([&](auto sc) {
+            constexpr int s = 1 - decltype(sc)::value;
+            if constexpr (!kPrefetch) load(e.app, s);
+            cpx<T> v[M], w[kBitc ? M : 1];
             static_for<0, M>([&](auto mc) { v[decltype(mc)::value] = vn[decltype(mc)::value]; });
-            if (pp + 1 < te.pair0 + te.npair) load_pencil<T, M>(vn, grid_of(pp + 1), S * nxy);
-        } else {
-            load_pencil<T, M>(v, grid_of(pp), S * nxy);  // z = S m + h
-        }
-        // FP32 up to 40^3: the orbital points are loaded before the transform, so that their
-        // latency overlaps it (at 48^3 the registers would halve the waves per SIMD; FP64
-        // loads them where they are used)
-        constexpr bool kHoist = kPrefetch && NZ <= 40;
-        cpx<T> xv[kHoist ? M : 1];
-        if constexpr (kHoist)
-            static_for<0, M>([&](auto kc) { xv[decltype(kc)::value] = xg[(size_t)decltype(kc)::value * nxy]; });
-        PencilSplit<S>::template fft<T, NZ, 1>(v, L.h);  // -> z = ob M + k
-        static_for<0, M>([&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            const double2 a = upd(v[k]);
-            double2 b;
-            if constexpr (kHoist)
-                b = upd(xv[k]);
-            else
-                b = upd(xg[(size_t)k * nxy]);
-            acc[k].x += (sy * f1) * (a.x * b.x - a.y * b.y);
-            acc[k].y += f1 * (a.x * b.y + a.y * b.x);
+            if constexpr (kPrefetch) {
+                if constexpr (s == 1)
+                    load(e.app, 0);
+                else if (i + 1 < end)
+                    load(entries[i + 1].app, 1);
+            }
+            PencilSplit<S>::template fft<T, NZ, 1>(v, L.h);  // -> z = ob M + k
+            if constexpr (kBitc) { ld_pencil<T, M>(w, chan(e.app, 1, s), ioff, S * nxy); PencilSplit<S>::template fft<T, NZ, 1>(w, L.h); }
+            __builtin_amdgcn_sched_barrier(0);  // the orbital points loaded earlier would spill
+            const cpx<T>* ph = occR + (size_t)e.occ * ng;
+            const cpx<T>* ch = chiR + (size_t)e.occ * ng;
+            static_for<0, M>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                const double2 a = upd(v[k]);
+                double2 b = a;
+                if constexpr (kBitc) b = upd(w[k]);
+                if constexpr (kBitc)
+                    q2[k] = cmadd(q2[k], a, make_double2(b.x, -b.y), -f1);
+                else
+                    q2[k].x -= f1 * (a.x * a.x + a.y * a.y);
+                if constexpr (s == 0) {
+                    // v_0 of the target: a, or -conj(b); conj(w_0): conj(b), or -a
+                    const double2 x = make_double2(rev ? -b.x : a.x, rev ? b.y : a.y);
+                    q4[k] = cmadd(q4[k], x, upd(ld<cpx<T>>(ph + (size_t)k * nxy, ooff)), f1);
+                    if constexpr (kBitc) {
+                        const double2 y = make_double2(rev ? -a.x : b.x, rev ? -a.y : -b.y), c = upd(ld<cpx<T>>(ch + (size_t)k * nxy, ooff));
+                        q5[k] = cmadd(q5[k], y, make_double2(c.x, -c.y), -f1);
+                    }
+                }
+                if constexpr (k % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+            });
         });
     }
     if (!L.valid) return;
-    double2* q = Q + ((size_t)te.app * 3 + d) * ng + o0;
-    static_for<0, M>([&](auto kc) {
-        constexpr int k = decltype(kc)::value;
-        const double2 a = q[(size_t)k * nxy];
-        q[(size_t)k * nxy] = make_double2(a.x + acc[k].x, a.y + acc[k].y);
-    });
+    auto add = [&](double2* q, const double2 (&acc)[M]) {
+        static_for<0, M>([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            const double2 a = q[(size_t)k * nxy];
+            q[(size_t)k * nxy] = make_double2(a.x + acc[k].x, a.y + acc[k].y);
+        });
+    };
+    add(Q2 + d * q2_slice + (size_t)te.app * ng + o0, q2);
+    add(Q4 + ((size_t)te.app * 3 + d) * ng + o0, q4);
+    if constexpr (kBitc) add(Q5 + ((size_t)te.app * 3 + d) * ng + o0, q5);
 }
 
 // Apply phase: W[t.app] += sum_p Z[p][0] phi_occ(p) + sum_d Z[p][1+d] Q4T[occ(p)][d]
@@ -390,28 +346,24 @@ void launch_za7_mid(int prec, const Geom& g, void* P, const void* occR, const Pa
 }
 
 void launch_za8_q(int prec, const Geom& g, const void* O, int bitc, const void* occR, const void* chiR,
-                  const PairEntry* pairs, const TargetEntry* targets, int ntargets, const double* fill, double* Q2,
-                  double* Q4, double* Q5, hipStream_t s)
+                  const PairEntry* entries, const TargetEntry* targets, int ntargets, const double* fill, double* Q2,
+                  size_t q2_slice, double* Q4, double* Q5, hipStream_t s)
 {
     const int nxy = g.n1 * g.n2;
-    const int nch = bitc ? 12 : 6;
     for_target_slices(ntargets, [&](int a, int n) {
 #define TCX_L(NZ)                                                                                              \
     {                                                                                                          \
-        /* 4 lanes per pencil for Q2 (2 would need 256 VGPRs); Q4/Q5 take 2 in FP32 (longer load runs) */  \
-        constexpr int SQ2 = SplitFor<NZ, 4>::value;                                                            \
-        constexpr int SQ45 = SplitFor<NZ, sizeof(T) == 8 ? 4 : 2>::value;                                     \
-        constexpr int P2 = PencilSplit<SQ2>::pencils, P4 = PencilSplit<SQ45>::pencils;                         \
-        hipLaunchKernelGGL((k_za8_q2<T, NZ, SQ2>), dim3((nxy + P2 - 1) / P2, n), dim3(kPencilBlock), 0, s,    \
-                           (const cpx<T>*)O, bitc, pairs, targets + a, fill, (double2*)Q2, nxy);               \
-        hipLaunchKernelGGL((k_za8_q45<T, NZ, SQ45>), dim3((nxy + P4 - 1) / P4, n, 3), dim3(kPencilBlock), 0, s, \
-                           (const cpx<T>*)O, nch, 0, 0, (const cpx<T>*)occR, pairs, targets + a, fill,        \
-                           (double2*)Q4, nxy);                                                                 \
+        constexpr int S = SplitFor<NZ, 4>::value;                                                              \
+        constexpr int PN = PencilSplit<S>::pencils;                                                            \
+        const dim3 grid((nxy + PN - 1) / PN, n, 3);                                                            \
         if (bitc)                                                                                              \
-            hipLaunchKernelGGL((k_za8_q45<T, NZ, SQ45>), dim3((nxy + P4 - 1) / P4, n, 3), dim3(kPencilBlock), 0, \
-                               s,                                                                              \
-                               (const cpx<T>*)O, nch, 6, 1, (const cpx<T>*)chiR, pairs, targets + a, fill,    \
-                               (double2*)Q5, nxy);                                                             \
+            hipLaunchKernelGGL((k_za8_q<T, NZ, S, true>), grid, dim3(kPencilBlock), 0, s, (const cpx<T>*)O,    \
+                               (const cpx<T>*)occR, (const cpx<T>*)chiR, entries, targets + a, fill,           \
+                               (double2*)Q2, q2_slice, (double2*)Q4, (double2*)Q5, nxy);                       \
+        else                                                                                                   \
+            hipLaunchKernelGGL((k_za8_q<T, NZ, S, false>), grid, dim3(kPencilBlock), 0, s, (const cpx<T>*)O,   \
+                               (const cpx<T>*)occR, (const cpx<T>*)chiR, entries, targets + a, fill,           \
+                               (double2*)Q2, q2_slice, (double2*)Q4, (double2*)Q5, nxy);                       \
     }
         TCX_Z_DISPATCH(prec, g, TCX_L);
 #undef TCX_L

@@ -50,29 +50,6 @@ struct PlaneRuns {
     __device__ __forceinline__ int base(int x) const { return (run[x] >> 16) - (run[x] & 0xff); }
 };
 
-// Grid and record accesses as (uniform base) + (32-bit lane offset in bytes): the base stays in
-// scalar registers and every element of a line takes scalar arithmetic only.  With a per-lane
-// pointer each of a line's 40 accesses needs a 64-bit vector address of its own, two
-// instructions and two registers (k_plane_Z at 40^3 took 226 registers, now about half).
-template <typename X>
-__device__ __forceinline__ X ld(const void* base, unsigned off)
-{
-    return *reinterpret_cast<const X*>((const char*)base + off);
-}
-template <typename T>
-__device__ __forceinline__ cpx<T> ld_nt(const void* base, unsigned off)
-{
-    typedef T v2 __attribute__((ext_vector_type(2)));
-    const v2 x = __builtin_nontemporal_load(reinterpret_cast<const v2*>((const char*)base + off));
-    return cpx<T>{x.x, x.y};
-}
-template <typename T>
-__device__ __forceinline__ void st_nt(void* base, unsigned off, cpx<T> x)
-{
-    typedef T v2 __attribute__((ext_vector_type(2)));
-    const v2 s = {x.re, x.im};
-    __builtin_nontemporal_store(s, reinterpret_cast<v2*>((char*)base + off));
-}
 template <typename T, int NZ>
 __device__ __forceinline__ void ld_column(cpx<T> (&v)[NZ], const cpx<T>* base, unsigned off, int cstride)
 {

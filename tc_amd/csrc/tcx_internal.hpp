@@ -236,8 +236,10 @@ void launch_za7_mid(int prec, const Geom& g, void* P, const void* occR, const Pa
                     const TargetEntry* targets, int ntargets, const double* fill, const double* dens,
                     long long dens_stride, double* qsum, double sc, hipStream_t s);
 void launch_za8_q(int prec, const Geom& g, const void* O, int bitc, const void* occR, const void* chiR,
-                  const PairEntry* pairs, const TargetEntry* targets, int ntargets, const double* fill, double* Q2,
-                  double* Q4, double* Q5, hipStream_t s);
+                  const PairEntry* entries, const TargetEntry* targets, int ntargets, const double* fill, double* Q2,
+                  size_t q2_slice, double* Q4, double* Q5, hipStream_t s);
+// a[0] += a[1] + a[2], slices of n complex values
+void launch_sum3(double* a, long long n, hipStream_t s);
 void launch_za8_apply(int prec, const Geom& g, const void* Z, const void* occR, const void* Q4T,
                       const PairEntry* pairs, const TargetEntry* targets, int ntargets, double* W, float* Wc,
                       hipStream_t s);

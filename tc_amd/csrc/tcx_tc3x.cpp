@@ -13,7 +13,6 @@
 // (kernels_zw.hip) and the [3a4,b5] block of tc3a2a4b2b5 (a8_kvaux).
 #include <algorithm>
 #include <cmath>
-#include <cstring>
 
 #include "tcx_terms.hpp"
 
@@ -25,8 +24,9 @@ namespace {
 constexpr size_t kRecordBudget = (size_t)3 << 30;
 constexpr long kTc3Targets = 32;
 
-// kPairsIrr*: as kPairsOcc*, with targets at the irreducible k of the k-mesh symmetry only
-enum PairKind { kPairsAppOcc = 0, kPairsOccOcc = 1, kPairsOccSameK = 2, kPairsIrrOcc = 3, kPairsIrrSameK = 4 };
+// kPairsIrrSameK: as kPairsOccSameK, with targets at the irreducible k of the k-mesh symmetry only;
+// kPairsQ: the q1-q2 set of q_pair_set
+enum PairKind { kPairsAppOcc = 0, kPairsOccSameK = 1, kPairsIrrSameK = 2, kPairsQ = 3 };
 
 ProdChan chan(const void* a, int a_sel, int a_mul, int a_off, int a_conj, const void* b, int b_sel, int b_mul,
               int b_off, int b_conj)
@@ -45,7 +45,7 @@ const PairSet& Context::pair_set(const std::vector<int>& nb, int kind, int chann
     auto key = std::make_tuple(kind == kPairsAppOcc ? nb : std::vector<int>(), kind * 1000 + channels * 2 + prec);
     auto it = pairsets.find(key);
     if (it != pairsets.end()) return it->second;
-    const bool irr = kind == kPairsIrrOcc || kind == kPairsIrrSameK;
+    const bool irr = kind == kPairsIrrSameK;
     const std::vector<PairItem> tg = kind == kPairsAppOcc ? applied_items(nb) : occupied_items(irr);
     const std::vector<PairItem> src = occupied_items();
     // the launch shape (tcx_set_launch_shape term 2) within the record budget, else automatic
@@ -57,6 +57,98 @@ const PairSet& Context::pair_set(const std::vector<int>& nb, int kind, int chann
     sc = std::min<long>(sc, (long)std::max<size_t>(1, src.size()));
     PairSet S;
     build_pairs(S, tg, src, tc, sc, kcart, kind == kPairsOccSameK || kind == kPairsIrrSameK);
+    auto res = pairsets.emplace(key, std::move(S));
+    return res.first->second;
+}
+
+// The q1-q2 pair set of tc3a2a4b2b5: records of nin input and 6 nin output channels, and per
+// target (q2,i2) the entries that k_za8_q sums.  The record of (q2,q1) also gives that of (q1,q2)
+// (role 1), so only the pairs i1 <= i2 are formed, in launches of a block of orbitals against
+// another: half the products and xy passes.  That needs K = q2-q1+G to be odd under the
+// exchange at every G of the pair density, which the Nyquist index of a basis that aliases is
+// not; such bases, and a k-mesh symmetry (sums at the irreducible q2 only), form every pair.
+// 40^3 FP32 BITC, 2x2x2 k, 12 bands: products and xy passes of the phase 20.7 -> 10.2 ms.
+const PairSet& Context::q_pair_set(int nin, int prec)
+{
+    const bool half = !sym_set && tc2x_two_channel();
+    auto key = std::make_tuple(std::vector<int>(), kPairsQ * 1000 + 2 * nin + prec);
+    auto it = pairsets.find(key);
+    if (it != pairsets.end()) return it->second;
+    const size_t es = prec == TCX_PREC_FP64 ? 16 : 8;
+    const std::vector<PairItem> src = occupied_items();
+    const long n = (long)src.size();
+    PairSet S;
+    if (!half) {
+        const long maxpairs = std::max<long>(1, (long)(kRecordBudget / ((size_t)7 * nin * N * es)));
+        const std::vector<PairItem> tg = occupied_items(sym_set);
+        const long want_t = shape_targets[2] > 0 ? shape_targets[2] : kTc3Targets;
+        const long tc = std::max<long>(1, std::min<long>({want_t, maxpairs, (long)std::max<size_t>(1, tg.size())}));
+        long sc = std::max<long>(1, maxpairs / tc);
+        if (shape_sources[2] > 0) sc = std::min<long>(sc, shape_sources[2]);
+        build_pairs(S, tg, src, tc, std::max<long>(1, std::min(sc, n)), kcart, false);
+        for (const Launch& L : S.launches) {
+            for (int p = 0; p < L.npairs; ++p) S.entries.push_back({p, S.pairs[L.pair0 + p].occ, 0, 0});
+            for (int t = 0; t < L.ntargets; ++t) S.targets[L.target0 + t].pair0 += L.pair0;
+        }
+    } else {
+        long B = (long)std::sqrt((double)kRecordBudget / ((double)7 * nin * N * es));
+        if (shape_targets[2] > 0) B = std::min(B, shape_targets[2]);
+        if (shape_sources[2] > 0) B = std::min(B, shape_sources[2]);
+        B = std::max<long>(1, std::min(B, std::max<long>(1, n)));
+        const long nblk = (n + B - 1) / B;
+        if (nblk > 0) B = (n + nblk - 1) / nblk;
+        for (long j0 = 0; j0 < n; j0 += B)
+            for (long i0 = 0; i0 <= j0; i0 += B) {
+                const long j1 = std::min(n, j0 + B), i1 = std::min(n, i0 + B);
+                const bool diag = i0 == j0;
+                const int kf = src[j0].k, kl = src[j1 - 1].k, qf = src[i0].k, ql = src[i1 - 1].k;
+                Launch L;
+                L.pair0 = (int)S.pairs.size();
+                L.target0 = (int)S.targets.size();
+                L.kq0 = (int)S.kq.size() / 3;
+                L.nkq = (kl - kf + 1) * (ql - qf + 1);
+                for (int k = kf; k <= kl; ++k)
+                    for (int q = qf; q <= ql; ++q) {
+                        for (int d = 0; d < 3; ++d) S.kq.push_back(kcart[3 * k + d] - kcart[3 * q + d]);
+                        S.kq_kq.push_back(k);
+                        S.kq_kq.push_back(q);
+                    }
+                // record of (j, i): row j of the block, its i from i0 on
+                std::vector<int> row(j1 - j0);
+                for (long j = j0; j < j1; ++j) {
+                    row[j - j0] = (int)S.pairs.size() - L.pair0;
+                    for (long i = i0; i < (diag ? j + 1 : i1); ++i)
+                        S.pairs.push_back({src[j].idx, src[i].idx,
+                                           L.kq0 + (src[j].k - kf) * (ql - qf + 1) + (src[i].k - qf), 0});
+                }
+                L.npairs = (int)S.pairs.size() - L.pair0;
+                for (long j = j0; j < j1; ++j) {
+                    TargetEntry te{src[j].idx, (int)S.entries.size(), 0, src[j].k};
+                    for (long i = i0; i < (diag ? j + 1 : i1); ++i)
+                        S.entries.push_back({row[j - j0] + (int)(i - i0), src[i].idx, 0, 0});
+                    if (diag)
+                        for (long m = j + 1; m < j1; ++m)
+                            S.entries.push_back({row[m - j0] + (int)(j - i0), src[m].idx, 1, 0});
+                    te.npair = (int)S.entries.size() - te.pair0;
+                    S.targets.push_back(te);
+                }
+                if (!diag)
+                    for (long i = i0; i < i1; ++i) {
+                        TargetEntry te{src[i].idx, (int)S.entries.size(), 0, src[i].k};
+                        for (long j = j0; j < j1; ++j)
+                            S.entries.push_back({row[j - j0] + (int)(i - i0), src[j].idx, 1, 0});
+                        te.npair = (int)S.entries.size() - te.pair0;
+                        S.targets.push_back(te);
+                    }
+                L.ntargets = (int)S.targets.size() - L.target0;
+                S.launches.push_back(L);
+                S.max_launch_pairs = std::max(S.max_launch_pairs, L.npairs);
+            }
+        upload(S.d_pairs, S.pairs.data(), S.pairs.size() * sizeof(PairEntry));
+        upload(S.d_kq, S.kq.data(), S.kq.size() * sizeof(double));
+    }
+    upload(S.d_targets, S.targets.data(), S.targets.size() * sizeof(TargetEntry));
+    upload(S.d_entries, S.entries.data(), S.entries.size() * sizeof(PairEntry));
     auto res = pairsets.emplace(key, std::move(S));
     return res.first->second;
 }
@@ -313,9 +405,9 @@ void Context::a8_occupied_phase(const std::vector<int>& nb, int prec)
 
     // (i) q1-q2 phase (:210-443): targets (q2,i2) x sources (q1,i1)
     const int nin = bitc ? 2 : 1;
-    d_Q2.ensure((size_t)n_occ * g64);
+    d_Q2.ensure((size_t)3 * n_occ * g64);  // a slice per direction, summed below
     d_Q4.ensure((size_t)3 * n_occ * g64);
-    launch_zero(d_Q2.p, (size_t)n_occ * g64, stream);
+    launch_zero(d_Q2.p, (size_t)3 * n_occ * g64, stream);
     launch_zero(d_Q4.p, (size_t)3 * n_occ * g64, stream);
     double* Q2 = (double*)d_Q2.p;
     double* Q4 = (double*)d_Q4.p;
@@ -326,7 +418,7 @@ void Context::a8_occupied_phase(const std::vector<int>& nb, int prec)
         Q5 = (double*)d_Q5.p;
     }
     {
-        const PairSet& S = pair_set(nb, sym_set ? kPairsIrrOcc : kPairsOccOcc, 7 * nin, prec);
+        const PairSet& S = q_pair_set(nin, prec);
         d_rec.ensure((size_t)std::max(1, S.max_launch_pairs) * 7 * nin * gT);
         int max_rows = 1;
         for (const Launch& L : S.launches) max_rows = std::max(max_rows, L.nkq);
@@ -351,10 +443,11 @@ void Context::a8_occupied_phase(const std::vector<int>& nb, int prec)
                                stream);
             });
             timed(2, np, [&] {  // z pass of FFT_backward fused with the q-sums
-                launch_za8_q(prec, geo, O, bitc ? 1 : 0, occR, chiR, pairs, targets, L.ntargets, fill, Q2, Q4,
-                             bitc ? Q5 : Q4, stream);
+                launch_za8_q(prec, geo, O, bitc ? 1 : 0, occR, chiR, (const PairEntry*)S.d_entries.p, targets,
+                             L.ntargets, fill, Q2, (size_t)n_occ * N, Q4, bitc ? Q5 : Q4, stream);
             });
         }
+        launch_sum3(Q2, (long long)n_occ * N, stream);
     }
 
     // (ii) [3a2]: T = FFT_forward(qsum_3a2) (:486-494), G=0 correction (:496-573)
@@ -640,13 +733,28 @@ void Context::apply_all(const int* nb_, const double* phi, double* h1, double* h
     for (int k = 0; k < nk; ++k) ncoef += (long long)nb_[k] * npw[k];
     const size_t bytes = (size_t)ncoef * 16;
     double* outs[3] = {h1, h2, tc ? h3 : nullptr};
-    for (double* o : outs) {
-        if (!o || bytes == 0) continue;
-        if (flags & TCX_FLAG_DEVICE_PTRS)
-            launch_zero(o, bytes, stream);
-        else
-            std::memset(o, 0, bytes);
+    const int nout = tc ? 3 : 2;
+    if (!(flags & TCX_FLAG_DEVICE_PTRS)) {
+        // Host pointers: one copy in, the terms on device buffers, one copy out per H_n phi.  Term by
+        // term each of the seven copied phi in and its own result out and added it on the host
+        // (with tc3a2a4b2b5's halved pair set, FP32 BITC, 24x24x18, 2x2x1 k, 6 bands: 2.8 -> 2.4 ms).
+        require(!g_capturing, TCX_ERR_STATE, "graph capture: term calls need TCX_FLAG_DEVICE_PTRS");
+        for (long long i = 0; i < ncoef * 2; ++i)
+            require(std::isfinite(phi[i]), TCX_ERR_ARG, "term: non-finite input coefficient");
+        const size_t slot = std::max<size_t>(16, bytes);
+        d_all.ensure((size_t)(1 + nout) * slot);
+        char* base = (char*)d_all.p;
+        if (bytes) TCX_HIP_CHECK(hipMemcpyAsync(base, phi, bytes, hipMemcpyHostToDevice, stream));
+        double* dev[3];
+        for (int n = 0; n < nout; ++n) dev[n] = (double*)(base + (size_t)(1 + n) * slot);
+        apply_all(nb_, (const double*)base, dev[0], dev[1], tc ? dev[2] : nullptr, prec, TCX_FLAG_DEVICE_PTRS);
+        for (int n = 0; n < nout; ++n)
+            if (bytes) TCX_HIP_CHECK(hipMemcpyAsync(outs[n], dev[n], bytes, hipMemcpyDeviceToHost, stream));
+        TCX_HIP_CHECK(hipStreamSynchronize(stream));
+        return;
     }
+    for (double* o : outs)
+        if (o && bytes) launch_zero(o, bytes, stream);
     kinetic(nb_, phi, h1, flags);
     if (!tc) {
         hf2h(nb_, phi, h2, flags);

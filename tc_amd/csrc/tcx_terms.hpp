@@ -67,7 +67,10 @@ struct PairSet {
     std::vector<int> kq_kq;  // (k, q) per row
     std::vector<Launch> launches;
     int max_launch_pairs = 0;
-    DBuf d_pairs, d_targets, d_kq;
+    // q-sum sets (q_pair_set): what a target sums, {launch-local record, source, role (1: the
+    // record of the reversed pair)}; their targets index these and not the pairs
+    std::vector<PairEntry> entries;
+    DBuf d_pairs, d_targets, d_kq, d_entries;
 };
 
 // A grid of a pair set: k-point and grid index (applied band or occupied orbital).
@@ -155,6 +158,7 @@ struct Context {
     DBuf d_occgradjobs;  // three OrbEntry (dir 0..2) per occupied orbital
     DBuf d_dc;       // divergence factor per k
     DBuf d_symjobs;  // SymRotJob per occupied orbital at a replica k
+    DBuf d_all;  // apply_all on host pointers: phi and the H_n phi
     DBuf d_phi_app, d_out, d_appR, d_appGrad, d_tmp64, d_W, d_pairbuf, d_ktab, d_work;
     DBuf d_Wc;  // compensation grids of the band-pair sums in d_W
 
@@ -330,6 +334,7 @@ struct Context {
 
     // three-body exchange terms and the assembly terms
     const PairSet& pair_set(const std::vector<int>& nb, int kind, int channels, int prec);
+    const PairSet& q_pair_set(int nin, int prec);
     std::vector<PairItem> applied_items(const std::vector<int>& nb) const;
     std::vector<PairItem> occupied_items(bool irreducible_only = false) const;
     void apply_local(const Plan& P, const ApplyIO& io, const double* V, double factor);
