@@ -162,7 +162,9 @@ __global__ __launch_bounds__(kPencilBlock) void k_za7_mid(cpx<T>* __restrict__ P
 // 40^3 FP32 BITC, 96 orbitals: 2.30 -> 1.67 us per ordered pair (3.7 TB/s of record reads; the
 // FP64 accumulators leave two waves per SIMD).
 // Two waves per SIMD where the accumulators leave room (the compiler took one for 36 points).
-template <typename T, int NZ, int S, bool kBitc>
+// kPart 0: all three sums; 1: Q2 only, 2: Q4 and Q5 only (s = 0), for BITC pencils of 15 points a
+// lane, whose three accumulators would leave one wave per SIMD.
+template <typename T, int NZ, int S, bool kBitc, int kPart>
 __global__ __launch_bounds__(kPencilBlock, (NZ / S <= (sizeof(T) == 4 ? 12 : 10) ? 2 : 1)) void k_za8_q(const cpx<T>* __restrict__ O, const cpx<T>* __restrict__ occR,
                                                         const cpx<T>* __restrict__ chiR,
                                                         const PairEntry* __restrict__ entries,
@@ -178,12 +180,14 @@ __global__ __launch_bounds__(kPencilBlock, (NZ / S <= (sizeof(T) == 4 ? 12 : 10)
     const int d = blockIdx.z;
     const size_t ng = (size_t)nxy * NZ;
     const size_t o0 = L.xy + (size_t)L.ob * M * nxy;
-    double2 q2[M], q4[M], q5[kBitc ? M : 1];
+    constexpr bool kQ2 = kPart != 2, kQ45 = kPart != 1;
+    constexpr int s_first = kQ2 ? 1 : 0;
+    double2 q2[kQ2 ? M : 1], q4[kQ45 ? M : 1], q5[kBitc && kQ45 ? M : 1];
     static_for<0, M>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
-        q2[k] = make_double2(0.0, 0.0);
-        q4[k] = make_double2(0.0, 0.0);
-        if constexpr (kBitc) q5[k] = make_double2(0.0, 0.0);
+        if constexpr (kQ2) q2[k] = make_double2(0.0, 0.0);
+        if constexpr (kQ45) q4[k] = make_double2(0.0, 0.0);
+        if constexpr (kBitc && kQ45) q5[k] = make_double2(0.0, 0.0);
     });
     // FP32 up to 40^3: the h = 0 pencil of the next (entry, s) step is loaded before this one is
     // transformed, the h = 1 pencil when v's registers are its own: 15.4 ms against 17.4 without
@@ -194,14 +198,14 @@ __global__ __launch_bounds__(kPencilBlock, (NZ / S <= (sizeof(T) == 4 ? 12 : 10)
     cpx<T> vn[M];
     auto load = [&](int rec, int s) { ld_pencil<T, M>(vn, chan(rec, 0, s), ioff, S * nxy); };  // z = S m + h
     const int end = te.pair0 + te.npair;
-    if (kPrefetch && te.npair > 0) load(entries[te.pair0].app, 1);
+    if (kPrefetch && te.npair > 0) load(entries[te.pair0].app, s_first);
 #pragma unroll 1
     for (int i = te.pair0; i < end; ++i) {
         const PairEntry e = entries[i];
         const double f1 = fill[e.occ];
         const bool rev = e.kq != 0;
-        static_for<0, 2>([&](auto sc) {
-            constexpr int s = 1 - decltype(sc)::value;
+        static_for<0, 1 + s_first>([&](auto sc) {
+            constexpr int s = s_first - decltype(sc)::value;
             if constexpr (!kPrefetch) load(e.app, s);
             cpx<T> v[M], w[kBitc ? M : 1];
             static_for<0, M>([&](auto mc) { v[decltype(mc)::value] = vn[decltype(mc)::value]; });
@@ -209,7 +213,7 @@ __global__ __launch_bounds__(kPencilBlock, (NZ / S <= (sizeof(T) == 4 ? 12 : 10)
                 if constexpr (s == 1)
                     load(e.app, 0);
                 else if (i + 1 < end)
-                    load(entries[i + 1].app, 1);
+                    load(entries[i + 1].app, s_first);
             }
             PencilSplit<S>::template fft<T, NZ, 1>(v, L.h);  // -> z = ob M + k
             if constexpr (kBitc) { ld_pencil<T, M>(w, chan(e.app, 1, s), ioff, S * nxy); PencilSplit<S>::template fft<T, NZ, 1>(w, L.h); }
@@ -221,11 +225,11 @@ __global__ __launch_bounds__(kPencilBlock, (NZ / S <= (sizeof(T) == 4 ? 12 : 10)
                 const double2 a = upd(v[k]);
                 double2 b = a;
                 if constexpr (kBitc) b = upd(w[k]);
-                if constexpr (kBitc)
+                if constexpr (kQ2 && kBitc)
                     q2[k] = cmadd(q2[k], a, make_double2(b.x, -b.y), -f1);
-                else
+                else if constexpr (kQ2)
                     q2[k].x -= f1 * (a.x * a.x + a.y * a.y);
-                if constexpr (s == 0) {
+                if constexpr (s == 0 && kQ45) {
                     // v_0 of the target: a, or -conj(b); conj(w_0): conj(b), or -a
                     const double2 x = make_double2(rev ? -b.x : a.x, rev ? b.y : a.y);
                     q4[k] = cmadd(q4[k], x, upd(ld<cpx<T>>(ph + (size_t)k * nxy, ooff)), f1);
@@ -246,9 +250,9 @@ __global__ __launch_bounds__(kPencilBlock, (NZ / S <= (sizeof(T) == 4 ? 12 : 10)
             q[(size_t)k * nxy] = make_double2(a.x + acc[k].x, a.y + acc[k].y);
         });
     };
-    add(Q2 + d * q2_slice + (size_t)te.app * ng + o0, q2);
-    add(Q4 + ((size_t)te.app * 3 + d) * ng + o0, q4);
-    if constexpr (kBitc) add(Q5 + ((size_t)te.app * 3 + d) * ng + o0, q5);
+    if constexpr (kQ2) add(Q2 + d * q2_slice + (size_t)te.app * ng + o0, q2);
+    if constexpr (kQ45) add(Q4 + ((size_t)te.app * 3 + d) * ng + o0, q4);
+    if constexpr (kBitc && kQ45) add(Q5 + ((size_t)te.app * 3 + d) * ng + o0, q5);
 }
 
 // Apply phase: W[t.app] += sum_p Z[p][0] phi_occ(p) + sum_d Z[p][1+d] Q4T[occ(p)][d]
@@ -356,14 +360,19 @@ void launch_za8_q(int prec, const Geom& g, const void* O, int bitc, const void* 
         constexpr int S = SplitFor<NZ, 4>::value;                                                              \
         constexpr int PN = PencilSplit<S>::pencils;                                                            \
         const dim3 grid((nxy + PN - 1) / PN, n, 3);                                                            \
-        if (bitc)                                                                                              \
-            hipLaunchKernelGGL((k_za8_q<T, NZ, S, true>), grid, dim3(kPencilBlock), 0, s, (const cpx<T>*)O,    \
-                               (const cpx<T>*)occR, (const cpx<T>*)chiR, entries, targets + a, fill,           \
-                               (double2*)Q2, q2_slice, (double2*)Q4, (double2*)Q5, nxy);                       \
-        else                                                                                                   \
-            hipLaunchKernelGGL((k_za8_q<T, NZ, S, false>), grid, dim3(kPencilBlock), 0, s, (const cpx<T>*)O,   \
-                               (const cpx<T>*)occR, (const cpx<T>*)chiR, entries, targets + a, fill,           \
-                               (double2*)Q2, q2_slice, (double2*)Q4, (double2*)Q5, nxy);                       \
+        constexpr bool kSplit = NZ / S > 12;                                                                   \
+        if (bitc) {                                                                                            \
+            hipLaunchKernelGGL((k_za8_q<T, NZ, S, true, kSplit ? 1 : 0>), grid, dim3(kPencilBlock), 0, s, (const cpx<T>*)O,        \
+                               (const cpx<T>*)occR, (const cpx<T>*)chiR, entries, targets + a, fill, (double2*)Q2,  \
+                               q2_slice, (double2*)Q4, (double2*)Q5, nxy);                                          \
+            if (kSplit)                                                                                        \
+                hipLaunchKernelGGL((k_za8_q<T, NZ, S, true, kSplit ? 2 : 0>), grid, dim3(kPencilBlock), 0, s, (const cpx<T>*)O,        \
+                               (const cpx<T>*)occR, (const cpx<T>*)chiR, entries, targets + a, fill, (double2*)Q2,  \
+                               q2_slice, (double2*)Q4, (double2*)Q5, nxy);                                      \
+        } else                                                                                                 \
+            hipLaunchKernelGGL((k_za8_q<T, NZ, S, false, 0>), grid, dim3(kPencilBlock), 0, s, (const cpx<T>*)O,        \
+                               (const cpx<T>*)occR, (const cpx<T>*)chiR, entries, targets + a, fill, (double2*)Q2,  \
+                               q2_slice, (double2*)Q4, (double2*)Q5, nxy);                                          \
     }
         TCX_Z_DISPATCH(prec, g, TCX_L);
 #undef TCX_L

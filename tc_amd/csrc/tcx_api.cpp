@@ -259,6 +259,7 @@ void Context::invalidate_states()
     density_valid = false;
     sym_jobs_valid = false;
     plans.clear();
+    band_jobs.clear();
     pairsets.clear();  // pair lists index the occupied orbitals and k-points
 }
 
@@ -545,6 +546,32 @@ void upload(DBuf& buf, const void* src, size_t bytes)
     if (bytes) TCX_HIP_CHECK(hipMemcpy(buf.p, src, bytes, hipMemcpyHostToDevice));
 }
 
+void upload_tables(DBuf& buf, std::initializer_list<TablePiece> pieces)
+{
+    size_t total = 0;
+    for (const TablePiece& t : pieces) total += (t.bytes + 255) / 256 * 256;
+    std::vector<char> host(total);
+    size_t o = 0;
+    for (const TablePiece& t : pieces) {
+        if (t.bytes) std::memcpy(host.data() + o, t.src, t.bytes);
+        o += (t.bytes + 255) / 256 * 256;
+    }
+    upload(buf, host.data(), total);
+    o = 0;
+    for (const TablePiece& t : pieces) {
+        t.view->p = (char*)buf.p + o;
+        o += (t.bytes + 255) / 256 * 256;
+    }
+}
+
+void PairSet::upload_pairs()
+{
+    upload_tables(tables, {{&d_pairs, pairs.data(), pairs.size() * sizeof(PairEntry)},
+                           {&d_targets, targets.data(), targets.size() * sizeof(TargetEntry)},
+                           {&d_kq, kq.data(), kq.size() * sizeof(double)},
+                           {&d_entries, entries.data(), entries.size() * sizeof(PairEntry)}});
+}
+
 void Context::ensure_occR(int prec)
 {
     if (occR_valid[prec]) return;
@@ -669,9 +696,7 @@ void build_pairs(PairSet& S, const std::vector<PairItem>& tg, const std::vector<
         }
     }
     for (const auto& L : S.launches) S.max_launch_pairs = std::max(S.max_launch_pairs, L.npairs);
-    upload(S.d_pairs, S.pairs.data(), S.pairs.size() * sizeof(PairEntry));
-    upload(S.d_targets, S.targets.data(), S.targets.size() * sizeof(TargetEntry));
-    upload(S.d_kq, S.kq.data(), S.kq.size() * sizeof(double));
+    S.upload_pairs();
 }
 
 std::vector<PairItem> Context::applied_items(const std::vector<int>& nb) const
@@ -693,6 +718,39 @@ std::vector<PairItem> Context::occupied_items(bool irreducible_only) const
     return v;
 }
 
+const BandJobs& Context::get_band_jobs(const std::vector<int>& nb)
+{
+    auto it = band_jobs.find(nb);
+    if (it != band_jobs.end()) return it->second;
+    BandJobSet J;
+    J.app_first.assign(nk + 1, 0);
+    J.app_coef.assign(nk + 1, 0);
+    for (int k = 0; k < nk; ++k) {
+        J.app_first[k + 1] = J.app_first[k] + nb[k];
+        J.app_coef[k + 1] = J.app_coef[k] + (long long)nb[k] * npw[k];
+    }
+    J.n_app = (int)J.app_first[nk];
+    // one scatter/gather job and one divergence job per applied band, in band order
+    std::vector<OrbEntry> appjobs, appgradjobs, app2jobs;
+    std::vector<DivEntry> divjobs;
+    for (int k = 0; k < nk; ++k)
+        for (int j = 0; j < nb[k]; ++j) {
+            const OrbEntry e{J.app_coef[k] + (long long)j * npw[k], npw[k], (int)pw_off[k], k, -1};
+            appjobs.push_back(e);
+            for (int d = 0; d < 3; ++d) appgradjobs.push_back({e.coef_off, e.npw, e.gidx_off, k, d});
+            for (int d : {-1, 3}) app2jobs.push_back({e.coef_off, e.npw, e.gidx_off, k, d});
+            if (zw_set && zw_k[k])  // the states given for a zero-weight k
+                divjobs.push_back({e.coef_off, zw_coef[k], npw[k], zw_n[k], zw_first[k], k});
+            else
+                divjobs.push_back({e.coef_off, occ_coef[k], npw[k], nocc[k], (int)occ_first[k], k});
+        }
+    upload_tables(J.tables, {{&J.d_appjobs, appjobs.data(), appjobs.size() * sizeof(OrbEntry)},
+                             {&J.d_appgradjobs, appgradjobs.data(), appgradjobs.size() * sizeof(OrbEntry)},
+                             {&J.d_app2jobs, app2jobs.data(), app2jobs.size() * sizeof(OrbEntry)},
+                             {&J.d_divjobs, divjobs.data(), divjobs.size() * sizeof(DivEntry)}});
+    return band_jobs.emplace(nb, std::move(J)).first->second;
+}
+
 // term 0: hf2x, 1: tc2x, kPlanJobs: the per-band jobs without the band pairs
 const Plan& Context::get_plan(const std::vector<int>& nb, int term, int prec)
 {
@@ -704,13 +762,7 @@ const Plan& Context::get_plan(const std::vector<int>& nb, int term, int prec)
     auto it = plans.find(key);
     if (it != plans.end()) return it->second;
     Plan P;
-    P.app_first.assign(nk + 1, 0);
-    P.app_coef.assign(nk + 1, 0);
-    for (int k = 0; k < nk; ++k) {
-        P.app_first[k + 1] = P.app_first[k] + nb[k];
-        P.app_coef[k + 1] = P.app_coef[k] + (long long)nb[k] * npw[k];
-    }
-    P.n_app = (int)P.app_first[nk];
+    static_cast<BandJobs&>(P) = get_band_jobs(nb);
     if (term == kPlanJobs) {
         // no pairs
     } else if (nspin == 1) {
@@ -729,26 +781,6 @@ const Plan& Context::get_plan(const std::vector<int>& nb, int term, int prec)
             for (size_t l = l0; l < P.launches.size(); ++l) P.launches[l].spin = s;
         }
     }
-    // one scatter/gather job and one divergence job per applied band, in band order
-    std::vector<OrbEntry> appjobs, appgradjobs, app2jobs;
-    std::vector<DivEntry> divjobs;
-    for (int k = 0; k < nk; ++k)
-        for (int j = 0; j < nb[k]; ++j) {
-            const OrbEntry e{P.app_coef[k] + (long long)j * npw[k], npw[k], (int)pw_off[k], k, -1};
-            appjobs.push_back(e);
-            for (int d = 0; d < 3; ++d) appgradjobs.push_back({e.coef_off, e.npw, e.gidx_off, k, d});
-            for (int d : {-1, 3}) app2jobs.push_back({e.coef_off, e.npw, e.gidx_off, k, d});
-            if (zw_set && zw_k[k])  // the states given for a zero-weight k
-                divjobs.push_back({e.coef_off, zw_coef[k], npw[k], zw_n[k], zw_first[k], k});
-            else
-                divjobs.push_back({e.coef_off, occ_coef[k], npw[k], nocc[k], (int)occ_first[k], k});
-        }
-    upload(P.d_appjobs, appjobs.data(), appjobs.size() * sizeof(OrbEntry));
-    upload(P.d_appgradjobs, appgradjobs.data(), appgradjobs.size() * sizeof(OrbEntry));
-    // hf2x and tc2x share a plan when their launch shapes agree
-    if (method != TCX_METHOD_HF && term != kPlanJobs)
-        upload(P.d_app2jobs, app2jobs.data(), app2jobs.size() * sizeof(OrbEntry));
-    upload(P.d_divjobs, divjobs.data(), divjobs.size() * sizeof(DivEntry));
     auto res = plans.emplace(key, std::move(P));
     return res.first->second;
 }

@@ -144,11 +144,8 @@ const PairSet& Context::q_pair_set(int nin, int prec)
                 S.launches.push_back(L);
                 S.max_launch_pairs = std::max(S.max_launch_pairs, L.npairs);
             }
-        upload(S.d_pairs, S.pairs.data(), S.pairs.size() * sizeof(PairEntry));
-        upload(S.d_kq, S.kq.data(), S.kq.size() * sizeof(double));
     }
-    upload(S.d_targets, S.targets.data(), S.targets.size() * sizeof(TargetEntry));
-    upload(S.d_entries, S.entries.data(), S.entries.size() * sizeof(PairEntry));
+    S.upload_pairs();
     auto res = pairsets.emplace(key, std::move(S));
     return res.first->second;
 }

@@ -5,6 +5,7 @@
 
 #include <complex>
 #include <functional>
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <tuple>
@@ -50,6 +51,19 @@ struct DBuf {
     void release();
 };
 
+// A slice of a packed table buffer.
+struct DView {
+    void* p = nullptr;
+};
+struct TablePiece {
+    DView* view;
+    const void* src;
+    size_t bytes;
+};
+// Copies the pieces into `buf` behind one another in one transfer (one allocation and one copy
+// for all tables of a plan) and points the views at them.
+void upload_tables(DBuf& buf, std::initializer_list<TablePiece> pieces);
+
 // One launch of the pair pipeline.
 struct Launch {
     int pair0 = 0, npairs = 0;      // slice of Plan::pairs; slot p of the pair buffer = pair0 + p
@@ -70,7 +84,9 @@ struct PairSet {
     // q-sum sets (q_pair_set): what a target sums, {launch-local record, source, role (1: the
     // record of the reversed pair)}; their targets index these and not the pairs
     std::vector<PairEntry> entries;
-    DBuf d_pairs, d_targets, d_kq, d_entries;
+    DBuf tables;
+    DView d_pairs, d_targets, d_kq, d_entries;
+    void upload_pairs();
 };
 
 // A grid of a pair set: k-point and grid index (applied band or occupied orbital).
@@ -83,14 +99,20 @@ struct PairItem {
 void build_pairs(PairSet& S, const std::vector<PairItem>& tg, const std::vector<PairItem>& src, long tc, long sc,
                  const std::vector<double>& kcart, bool same_k);
 
-struct Plan : PairSet {
+// What the terms read per applied band, shared by the plans of the same band counts.
+struct BandJobs {
     std::vector<long long> app_first, app_coef;  // per k: first applied orbital, coefficient offset
     int n_app = 0;
-    DBuf d_appjobs;      // OrbEntry per applied band (band order)
-    DBuf d_appgradjobs;  // three OrbEntry (dir 0..2) per applied band
-    DBuf d_app2jobs;     // two OrbEntry (phi, |k+G|^2 phi) per applied band
-    DBuf d_divjobs;      // DivEntry per applied band
+    DView d_appjobs;      // OrbEntry per applied band (band order)
+    DView d_appgradjobs;  // three OrbEntry (dir 0..2) per applied band
+    DView d_app2jobs;     // two OrbEntry (phi, |k+G|^2 phi) per applied band
+    DView d_divjobs;      // DivEntry per applied band
 };
+struct BandJobSet : BandJobs {
+    DBuf tables;
+};
+
+struct Plan : PairSet, BandJobs {};
 
 // synchronous host -> device copy into a growing buffer
 void upload(DBuf& buf, const void* src, size_t bytes);
@@ -187,6 +209,8 @@ struct Context {
     bool sets_valid[2] = {false, false}, a_sets_valid[2] = {false, false};
     DBuf d_occ2jobs, d_occ5jobs;  // OrbEntry (phi, L) and (phi, L, g_d) per occupied orbital
     std::map<std::tuple<std::vector<int>, long, long>, Plan> plans;
+    std::map<std::vector<int>, BandJobSet> band_jobs;  // cleared with the plans that view them
+    const BandJobs& get_band_jobs(const std::vector<int>& nb);
     // pair sets of the three-body exchange terms, keyed by (applied bands, kind)
     std::map<std::tuple<std::vector<int>, int>, PairSet> pairsets;
     DBuf d_qsum, d_qsumT, d_rec, d_Q2, d_Q4, d_Q5, d_Q4T, d_Q5T, d_appR64, d_chans, d_aux, d_local;

@@ -113,6 +113,7 @@ void Context::set_zero_weight(const double* kweight, const double* skv, const in
     occR_valid[0] = occR_valid[1] = false;
     chiR_valid[0] = chiR_valid[1] = false;
     plans.clear();  // divergence jobs address the new states
+    band_jobs.clear();
     d_phi_occ = std::move(nphi);
     if (bitc) d_chi_occ = std::move(nchi);
     d_fill = std::move(nfill);
