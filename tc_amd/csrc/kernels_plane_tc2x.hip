@@ -267,25 +267,18 @@ __global__ __launch_bounds__((Tc2xWg<NP>::threads), 2) void k_plane_tc2x_C(
     auto plane_of = [&](int pp) { return rec + ((size_t)pp * 2 * nz + z) * pc.cstride; };  // uniform
     const unsigned off = (unsigned)(r * nz * pc.cstride + t) * sizeof(cpx<float>);         // pair r/2, channel r&1
     const unsigned koff = (unsigned)(r * NP + t) * sizeof(Ket);
-#ifndef V_PRE
-#define V_PRE 1
-#endif
-#ifndef V_SB
-#define V_SB 2
-#endif
     cpx<float> v[NP];
-    if (V_PRE && r < R && te.pair0 + r / 2 < pend) load_row<float, NP>(v, plane_of(te.pair0), off, runs, t);
+    if (r < R && te.pair0 + r / 2 < pend) load_row<float, NP>(v, plane_of(te.pair0), off, runs, t);
 #pragma unroll 1
     for (int p0 = te.pair0; p0 < pend; p0 += S) {
         const bool on = r < R && p0 + r / 2 < pend, next = r < R && p0 + S + r / 2 < pend;
-        if (!V_PRE && on) load_row<float, NP>(v, plane_of(p0), off, runs, t);
         if (on) fft<float, NP, 1>(v);
         rows_to_cols<float, NP>(tile, v, row, t, on);
         if (on) {
             fft<float, NP, 1>(v);
             tile_put_col<float, NP>(tile, v, t);  // column t was read by this thread alone
         }
-        if (V_PRE && next) load_row<float, NP>(v, plane_of(p0 + S), off, runs, t);
+        if (next) load_row<float, NP>(v, plane_of(p0 + S), off, runs, t);
         __syncthreads();
         const int ns = pend - p0 < S ? pend - p0 : S;
         if (r < R)
@@ -312,7 +305,7 @@ __global__ __launch_bounds__((Tc2xWg<NP>::threads), 2) void k_plane_tc2x_C(
                             acc[1 + d][i].y += f * (double)w.im;
                         });
                     }
-                    if constexpr (V_SB > 0 && i % (V_SB > 0 ? V_SB : 1) == V_SB - 1) __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
                 });
             }
         __syncthreads();
