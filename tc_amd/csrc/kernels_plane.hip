@@ -43,13 +43,13 @@ using PT = float;  // precision of the pair records
 // Plane-group-fastest order also keeps the record writes in flight close together: a
 // plane-slowest order, which gives each XCD a fixed set of planes too, took 139 ms.
 template <typename T, int NP>
-__global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_A(const cpx<T>* __restrict__ phiR_app,
+__global__ __launch_bounds__((PlaneWgA<T, NP>::threads), 2) void k_plane_A(const cpx<T>* __restrict__ phiR_app,
                                                                      const cpx<T>* __restrict__ phiR_occ,
                                                                      const PairEntry* __restrict__ pairs, int nsrc,
                                                                      const int* __restrict__ runs, PlaneCols pc,
                                                                      cpx<T>* __restrict__ rec, int nz)
 {
-    using Wg = PlaneWg<T, NP>;
+    using Wg = PlaneWgA<T, NP>;
     __shared__ PlaneTile<T, NP> tiles[Wg::R];
     const int ngrp = (nz + Wg::R - 1) / Wg::R, per = (nsrc * ngrp + 7) & ~7;
     const int tg = blockIdx.x / per, i = blockIdx.x - tg * per;
@@ -132,12 +132,12 @@ __global__ __launch_bounds__(kPencilBlock, 2) void k_plane_Z(cpx<T>* __restrict_
 // 40^3) with whole lines per lane: split lines (4 lanes each, the accumulators by line) cost
 // twice the instructions and ran 2.7 times longer.
 template <typename T, int NP>
-__global__ __launch_bounds__((PlaneWg<T, NP>::threads), 2) void k_plane_C(
+__global__ __launch_bounds__((PlaneWgC<T, NP>::threads), 2) void k_plane_C(
     const cpx<T>* __restrict__ rec, const cpx<T>* __restrict__ phiR_occ, const PairEntry* __restrict__ pairs,
     const TargetEntry* __restrict__ targets, const int* __restrict__ runs, PlaneCols pc,
     const double* __restrict__ fill, cpx<double>* __restrict__ W, float2* __restrict__ Wc, int nz)
 {
-    using Wg = PlaneWg<T, NP>;
+    using Wg = PlaneWgC<T, NP>;
     constexpr int R = Wg::R, ROWS = Wg::rows;
     __shared__ PlaneTile<T, NP> tiles[R];
     const int z = blockIdx.x;
@@ -204,7 +204,7 @@ PlaneShape plane_shape(int n1)
     PlaneShape ps{1, 256};
 #define TCX_L(NP)                                                                              \
     {                                                                                          \
-        using Wg = PlaneWg<PT, NP>;                                                             \
+        using Wg = PlaneWgC<PT, NP>;                                                             \
         const int by_lds = (160 * 1024) / (Wg::R * Wg::tile_bytes), by_waves = 8 / (Wg::threads / 64); \
         ps = {Wg::R, 256 * (by_lds < by_waves ? by_lds : by_waves)};                           \
     }
@@ -219,7 +219,7 @@ void launch_plane_A(const Geom& g, const void* app, const void* occ, const PairE
     if (ntargets == 0 || nsrc == 0) return;
 #define TCX_L(NP)                                                                                                \
     {                                                                                                            \
-        using Wg = PlaneWg<PT, NP>;                                                                               \
+        using Wg = PlaneWgA<PT, NP>;                                                                               \
         const unsigned per = ((unsigned)((g.n3 + Wg::R - 1) / Wg::R) * nsrc + 7) / 8 * 8;                        \
         hipLaunchKernelGGL((k_plane_A<PT, NP>), dim3(per * ntargets), dim3(Wg::threads), 0, s, (const cpx<PT>*)app, \
                            (const cpx<PT>*)occ, pairs, nsrc, pc.run, pc, (cpx<PT>*)rec, g.n3);                   \
@@ -260,7 +260,7 @@ void launch_plane_C(const Geom& g, const void* rec, const void* occ, const PairE
     if (ntargets > 65535) throw Error(TCX_ERR_INTERNAL, "plane pipeline: too many targets in one launch");
 #define TCX_L(NP)                                                                                                \
     {                                                                                                            \
-        using Wg = PlaneWg<PT, NP>;                                                                               \
+        using Wg = PlaneWgC<PT, NP>;                                                                               \
         hipLaunchKernelGGL((k_plane_C<PT, NP>), dim3(g.n3, ntargets), dim3(Wg::threads), 0, s,                    \
                            (const cpx<PT>*)rec, (const cpx<PT>*)occ, pairs, targets, pc.run, pc, fill,             \
                            (cpx<double>*)W, (float2*)Wc, g.n3);                                                  \

@@ -100,7 +100,9 @@ void launch_gather_tc2x(const double* W, const int* gindex, const OrbEntry* jobs
 namespace {
 
 // Workgroup of pass C: R tiles, tile 2 s + c = channel c of pair s of the group.  At most 8 plane
-// rows a thread (four FP64 accumulators per point); else as PlaneWg.
+// rows a thread (four FP64 accumulators per point), two wavefronts or more where a plane has
+// them, and more tiles only for clearly more of the lanes in use (FP32, per apply: 16^3 0.16 ->
+// 0.13 ms with 8 tiles for 4; 20^3 1.61 -> 1.01 ms with 6 for 16).
 template <int NP>
 struct Tc2xWg {
     static constexpr int tile_bytes = (int)sizeof(PlaneTile<float, NP>);
@@ -109,12 +111,12 @@ struct Tc2xWg {
         int best = 0;
         double best_score = 0.0;
         for (int r = 2; r <= 16 && r <= NP && r * NP <= 512 && r * tile_bytes <= 160 * 1024; r += 2) {
-            if (r * 8 < NP) continue;
+            if (r * 8 < NP || (NP >= 16 && r * NP <= 64)) continue;
             const int waves = (r * NP + 63) / 64;
             const int per_cu = (160 * 1024) / (r * tile_bytes) * waves;
             const double score = double(r * NP) / (64 * waves) * (per_cu >= 8 ? 1.0 : per_cu / 8.0) *
                                  (per_cu >= 2 * waves ? 1.0 : 0.8);  // one workgroup alone waits at its barriers
-            if (score > best_score + 1e-9) {
+            if (score > best_score + 0.145) {
                 best_score = score;
                 best = r;
             }
@@ -160,11 +162,11 @@ __global__ __launch_bounds__(256) void k_plane_tc_table(cpx<float>* __restrict__
 // Pass A: R planes of one pair, rho and then tau through the same tiles (both at once would take
 // the registers of a wave per SIMD from 36 points a line on).
 template <int NP>
-__global__ __launch_bounds__((PlaneWg<float, NP>::threads), 2) void k_plane_tc2x_A(
+__global__ __launch_bounds__((PlaneWgA<float, NP>::threads), 2) void k_plane_tc2x_A(
     const Bra* __restrict__ app, const Bra* __restrict__ bra, const PairEntry* __restrict__ pairs, int nsrc,
     const int* __restrict__ runs, PlaneCols pc, cpx<float>* __restrict__ rec, int nz)
 {
-    using Wg = PlaneWg<float, NP>;
+    using Wg = PlaneWgA<float, NP>;
     __shared__ PlaneTile<float, NP> tiles[Wg::R];
     const int ngrp = (nz + Wg::R - 1) / Wg::R, per = (nsrc * ngrp + 7) & ~7;  // as k_plane_A
     const int tg = blockIdx.x / per, i = blockIdx.x - tg * per;
@@ -357,7 +359,7 @@ void launch_plane_tc2x_A(const Geom& g, const void* app, const void* bra, const 
     if (ntargets == 0 || nsrc == 0) return;
 #define TCX_L(NP)                                                                                             \
     {                                                                                                         \
-        using Wg = PlaneWg<float, NP>;                                                                        \
+        using Wg = PlaneWgA<float, NP>;                                                                        \
         const unsigned per = ((unsigned)((g.n3 + Wg::R - 1) / Wg::R) * nsrc + 7) / 8 * 8;                     \
         hipLaunchKernelGGL((k_plane_tc2x_A<NP>), dim3(per * ntargets), dim3(Wg::threads), 0, s, (const Bra*)app, \
                            (const Bra*)bra, pairs, nsrc, pc.run, pc, (cpx<float>*)rec, g.n3);                 \

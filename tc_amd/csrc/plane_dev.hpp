@@ -6,32 +6,70 @@
 
 namespace tcx {
 
-// Workgroup of the plane passes: R tiles (planes of a pair in pass A, pairs of a plane in
-// pass C) of NP lines each, line t of tile r on thread r NP + t.  R fills the wavefronts best
-// among those that leave 8 wavefronts (2 per SIMD) of workgroups in a CU's 160 KB of LDS, with
-// at most 16 accumulators a thread (a single 48-line tile would hold 48 of them: 48^3 ran at two
-// thirds of the z-first speed).
+// Workgroups of the plane passes: R tiles (planes of a pair in pass A, pairs of a plane in
+// pass C) of NP lines each, line t of tile r on thread r NP + t.
 template <typename T, int NP>
 struct PlaneWg {
     static constexpr int tile_bytes = (int)sizeof(PlaneTile<T, NP>);
+    // tiles that fill w wavefronts, and the share of the lanes that they use in percent
+    static constexpr int fit(int w) { return 64 * w / NP < NP ? 64 * w / NP : NP; }
+    static constexpr int fill(int w)
+    {
+        const int lanes = fit(w) * NP;
+        return 100 * lanes / (64 * ((lanes + 63) / 64));
+    }
+};
+
+// Pass A has no work that tiles share: the fewest wavefronts whose lanes are 84% used, so that
+// a workgroup waits for little but its own transpose.  Against filling the lanes best (FP32, per
+// apply): 36^3 hf2x 4.4 -> 3.9 ms, tc2x 13.0 -> 10.4 ms with 3 planes for 7; 32^3, 30^3 two
+// planes 31 and 1.7 ms against 42 and 2.3 ms with eight.
+template <typename T, int NP>
+struct PlaneWgA : PlaneWg<T, NP> {
+    using B = PlaneWg<T, NP>;
     static constexpr int pick()
     {
-        int best = (NP + 15) / 16;
-        double best_score = 0.0;
-        for (int r = (NP + 15) / 16; r <= 16 && r * NP <= 256 && r * tile_bytes <= 80 * 1024; ++r) {
-            const int waves = (r * NP + 63) / 64;
-            const int per_cu = (160 * 1024) / (r * tile_bytes) * waves;
-            const double score = double(r * NP) / (64 * waves) * (per_cu >= 8 ? 1.0 : per_cu / 8.0);
-            if (score > best_score + 1e-9) {
-                best_score = score;
+        int best = 0, best_fill = 0;
+        for (int w = 1; w <= 4; ++w) {
+            const int r = B::fit(w);
+            if (r < 1 || r * B::tile_bytes > 80 * 1024 || best_fill >= 84) continue;
+            if (B::fill(w) > best_fill) {
                 best = r;
+                best_fill = B::fill(w);
             }
         }
         return best;
     }
     static constexpr int R = pick();
     static constexpr int threads = ((R * NP + 63) / 64) * 64;
-    static constexpr int rows = (NP + R - 1) / R;  // plane rows a thread sums in pass C
+    static_assert(R >= 1 && threads <= 256, "plane pass A workgroup");
+};
+
+// Pass C sums the points of a plane over its R tiles, so every tile more also takes accumulators
+// off a thread: two wavefronts, and more only where they use over a tenth more of their lanes
+// (36^3: 7 pairs, 48^3: 4).  One wavefront, 15 and 16 accumulators a thread, took 4.1 ms at
+// 30^3 and 67 ms at 32^3 where two take 2.3 and 39 ms; 24^3 with one 21, with two 11.3, with
+// four 12.0 ms; 40^3 with two 21, with four 23 ms.
+template <typename T, int NP>
+struct PlaneWgC : PlaneWg<T, NP> {
+    using B = PlaneWg<T, NP>;
+    static constexpr int pick()
+    {
+        int best = 0, best_fill = -11;
+        for (int w = 2; w <= 4; ++w) {
+            const int r = B::fit(w);
+            if (r < 1 || r * B::tile_bytes > 80 * 1024) continue;
+            if (B::fill(w) > best_fill + 10) {
+                best = r;
+                best_fill = B::fill(w);
+            }
+        }
+        return best;
+    }
+    static constexpr int R = pick();
+    static constexpr int threads = ((R * NP + 63) / 64) * 64;
+    static constexpr int rows = (NP + R - 1) / R;  // plane rows a thread sums
+    static_assert(R >= 1 && R <= NP && rows <= 16 && threads <= 256, "plane pass C workgroup");
 };
 
 // The runs of a column set, read once per workgroup into scalar registers.
