@@ -403,8 +403,9 @@ int tcx_get_record_columns(tcx_context *ctx, int term, double *columns);
 int tcx_set_launch_shape(tcx_context *ctx, int term, long targets, long sources);
 
 /* Per-kernel-class timing with HIP events on the context's stream.
- * Classes: 0 pair pass A (z-pencils), 1 pair pass B (xy-planes),
- * 2 pair pass C (z-pencils + accumulate), 3 orbital/final transforms.
+ * Classes: 0 the first pair pass (z pencils; xy planes in the plane-first order), 1 the middle
+ * one (xy planes; z pencils of the support columns), 2 the last one with the accumulation
+ * (z pencils; xy planes), 3 orbital/final transforms.
  * out_ms[c] = summed duration (ms), out_launches[c] = number of launches,
  * out_pairs[c] = pairs processed by that class. */
 int tcx_enable_timing(tcx_context *ctx, int on);
