@@ -210,7 +210,7 @@ void Context::kernel_grad(int term, int nbins, double width, double* dE_dK, doub
             for (int d = 0; d < 3; ++d) ch.push_back(ProdChan{gradR, chiR, 1, 3, d, 1, 0, 1, 0, 0});  // tau_d
         }
         upload(d_chans, ch.data(), ch.size() * sizeof(ProdChan));
-        const PairSet& S = pair_set(nocc, 1, C, prec);  // occupied x occupied
+        const PairSet& S = pair_set(nocc, kPairsOccOcc, C, prec);
         d_rec.ensure((size_t)std::max(1, S.max_launch_pairs) * C * gT);
         const double NkV = num_kpoints * volume;
         double c = tc2 ? -1.0 / NkV : -4.0 * kPiHost / NkV;  // two_body_factor of tc2x / hf2x

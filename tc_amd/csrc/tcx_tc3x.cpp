@@ -24,10 +24,6 @@ namespace {
 constexpr size_t kRecordBudget = (size_t)3 << 30;
 constexpr long kTc3Targets = 32;
 
-// kPairsIrrSameK: as kPairsOccSameK, with targets at the irreducible k of the k-mesh symmetry only;
-// kPairsQ: the q1-q2 set of q_pair_set
-enum PairKind { kPairsAppOcc = 0, kPairsOccSameK = 1, kPairsIrrSameK = 2, kPairsQ = 3 };
-
 ProdChan chan(const void* a, int a_sel, int a_mul, int a_off, int a_conj, const void* b, int b_sel, int b_mul,
               int b_off, int b_conj)
 {
@@ -38,7 +34,7 @@ ProdChan chan(const void* a, int a_sel, int a_mul, int a_off, int a_conj, const 
 
 // Pair set of one kind, with launches sized so that `channels` record grids
 // per pair stay under kRecordBudget.
-const PairSet& Context::pair_set(const std::vector<int>& nb, int kind, int channels, int prec)
+const PairSet& Context::pair_set(const std::vector<int>& nb, PairKind kind, int channels, int prec)
 {
     const size_t es = prec == TCX_PREC_FP64 ? 16 : 8;
     // only the (k,j) x (q,i) kind depends on the applied bands

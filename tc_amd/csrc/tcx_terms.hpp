@@ -89,6 +89,11 @@ struct PairSet {
     void upload_pairs();
 };
 
+// Pair sets of the three-body terms and of the kernel gradients: (k,j) x (q,i), occupied x occupied,
+// occupied x occupied of the same k (kPairsIrrSameK: targets at the irreducible k of the k-mesh
+// symmetry only), and the q1-q2 set of q_pair_set
+enum PairKind { kPairsAppOcc, kPairsOccOcc, kPairsOccSameK, kPairsIrrSameK, kPairsQ };
+
 // A grid of a pair set: k-point and grid index (applied band or occupied orbital).
 struct PairItem {
     int k, idx;
@@ -357,7 +362,7 @@ struct Context {
     void tc3_local(int which, const int* nb, const double* phi, double* out, int prec, unsigned flags);
 
     // three-body exchange terms and the assembly terms
-    const PairSet& pair_set(const std::vector<int>& nb, int kind, int channels, int prec);
+    const PairSet& pair_set(const std::vector<int>& nb, PairKind kind, int channels, int prec);
     const PairSet& q_pair_set(int nin, int prec);
     std::vector<PairItem> applied_items(const std::vector<int>& nb) const;
     std::vector<PairItem> occupied_items(bool irreducible_only = false) const;
