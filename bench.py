@@ -30,8 +30,9 @@ sys.path.insert(0, ROOT)
 
 METRIC = "pair-FFT operator applies/s + HBM GB/s: FP32-split vs FP64 at ΔE<1e-6 Ha"
 HBM_PEAK_GBS = 8000.0
-# timing classes of a plane-first apply (FP32-split hf2x, and tc2x where its bases do not alias)
+# timing classes of a plane-first apply (FP32-split hf2x) and of a z-first one (tc2x)
 CLASS_NAMES = ["pass_A_xyplane", "pass_Z_zpencil", "pass_C_xyplane_acc", "orbital_and_final_fft"]
+Z_FIRST_NAMES = ["pass_A_zpencil", "pass_B_xyplane", "pass_C_zpencil_acc", "orbital_and_final_fft"]
 
 
 def log(msg):
@@ -670,9 +671,9 @@ def bench_tc_legs(eng, log, tc_steps):
             of its dominant pass; one FP64 apply after a warm-up; energy and per-band errors;
       tc3a3b3b4b6, tc3a2a4b2b5: FP32-split first apply (occupied-set work included), repeated
             apply (occupied-set q-sums reused), FP64 first apply; energy errors.
-    Algorithmic values per tc2x pair and pass (N points, R record values per channel, 8 B each):
-    pass A reads chi_qi and L chi_qi and writes 2 channels (2 N + 2 R), pass Z reads and writes
-    them (4 R), pass C reads them and phi_qi, L phi_qi and the three g_qi,d (2 R + 5 N)."""
+    Algorithmic bytes per tc2x pair and pass (N points, 8 B per FP32 complex value): pass A
+    reads chi_qi and writes 4 record channels (5 N 8 B), pass B reads and writes 4 channels
+    (8 N 8 B), pass C reads 4 channels and the 4 grids of phi_qi and grad phi_qi (8 N 8 B)."""
     from tc_amd import energy as E
     from tc_amd import system as S
     from tc_amd import tcx
@@ -731,25 +732,23 @@ def bench_tc_legs(eng, log, tc_steps):
     h64 = d_out.download(np.complex128)
     e32 = E.term_energy(sys_, h32, 2, left=True)
     e64 = E.term_energy(sys_, h64, 2, left=True)
-    apply("hf2x", tcx.PREC_FP32)  # same bases, same support columns
-    n_rec = eng.record_columns("hf2x") * sys_.n[2]
-    words = [2 * N + 2 * n_rec, 4 * n_rec, 2 * n_rec + 5 * N]
+    words = [5, 8, 8]   # grid values moved per pair in passes A, B, C
     dom = int(np.argmax(ms[:3]))
     avg_ms = ms[dom] / max(1, launches[dom])
     ppl = kpairs[dom] / max(1, launches[dom])
-    bpl = words[dom] * 8 * ppl
+    bpl = words[dom] * N * 8 * ppl
     fp32_s = float(np.median(t32))
     res["tc2x"] = {
         "fp32_ms": fp32_s * 1e3, "fp64_ms": t64 * 1e3, "fp32_over_fp64": t64 / fp32_s,
         "fp32_pairs_per_s": pairs / fp32_s, "E_fp64_Ha": [float(e64.real), float(e64.imag)],
         "dE_Ha": float(abs(e32 - e64)), "per_band_rel_max": per_band(h32, h64),
-        "pipeline_algorithmic_GBps": sum(words) * 8 * pairs / fp32_s / 1e9,
+        "pipeline_algorithmic_GBps_21NBc": 21 * N * 8 * pairs / fp32_s / 1e9,
         "roofline": {"bound": "hbm", "achieved": bpl / (avg_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": bpl / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                     "traffic": read_traffic("tc2x_" + CLASS_NAMES[dom], ppl),
-                     "kernel": "tc2x_" + CLASS_NAMES[dom], "avg_launch_ms": avg_ms, "pairs_per_launch": ppl,
+                     "traffic": read_traffic("tc2x_" + Z_FIRST_NAMES[dom], ppl),
+                     "kernel": "tc2x_" + Z_FIRST_NAMES[dom], "avg_launch_ms": avg_ms, "pairs_per_launch": ppl,
                      "algorithmic_bytes_per_launch": bpl},
-        "class_ms_per_apply": {CLASS_NAMES[c]: float(ms[c]) / tc_steps for c in range(4)},
+        "class_ms_per_apply": {Z_FIRST_NAMES[c]: float(ms[c]) / tc_steps for c in range(4)},
     }
     # ---- three-body exchange terms
     res["three_body"] = {}

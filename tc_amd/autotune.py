@@ -62,7 +62,7 @@ def three_body_candidates(n_targets, n_sources):
 def tune(eng, sys_, term, nb, d_phi, d_out, precision, candidates=None, log=print, samples=SAMPLES):
     """Time `samples` full applies per candidate shape (after one untimed apply that
     builds the plan and warms the caches) and return (best_shape, {shape: median s})."""
-    channels = 2 if term == "tc2x" else 1  # records of tc2x's two-channel form
+    channels = 4 if term == "tc2x" else 1
     if candidates is None:
         if TERMS[term] == 2:
             candidates = three_body_candidates(int(np.sum(nb)), int(np.sum(sys_.nocc)))
@@ -133,7 +133,7 @@ def main(argv=None):
 
     # a short candidate list per term keeps a workload's sweep within minutes
     short = {"hf2x": [(48, 48), (96, 32), (96, 48), (96, 96), (192, 48), (192, 96)],
-             "tc2x": [(32, 32), (32, 64), (64, 32), (64, 48), (96, 32), (96, 48), (128, 32)],
+             "tc2x": [(16, 32), (32, 32), (32, 64), (64, 16), (64, 32), (96, 16), (128, 8), (128, 16)],
              "tc3a2a4b2b5": [(16, 16), (32, 8), (32, 16), (64, 8), (64, 16)],
              "tc3a3b3b4b6": [(16, 16), (32, 8), (32, 16), (64, 8), (64, 16)]}
 

@@ -28,7 +28,6 @@ SOURCES = [
     "csrc/kernels_fft.hip",
     "csrc/kernels_hf2x.hip",
     "csrc/kernels_plane.hip",
-    "csrc/kernels_plane_tc2x.hip",
     "csrc/kernels_tc2x.hip",
     "csrc/kernels_local.hip",
     "csrc/kernels_tc3x.hip",

@@ -67,10 +67,9 @@ __device__ __forceinline__ void add_partial(double2* w, float2* wc, double are, 
 
 // Grid and record accesses as (uniform base) + (32-bit lane offset in bytes): the base stays in
 // scalar registers and every element of a line takes scalar arithmetic only.  With a per-lane
-// pointer each of a line's 40 accesses needs a 64-bit vector address of its own: an
-// instruction and two registers each, which spill where a kernel holds two lines
-// (k_plane_tc2x_Z).  Where one line fits either way the pointers can be the faster form
-// (k_plane_A), so a kernel takes what it was measured with.
+// pointer each of a line's accesses needs a 64-bit vector address of its own: an instruction and
+// two registers each.  hf2x in FP64 at 36^3 (3x3x2 k) took 20.53 ms this way against 20.88, but
+// k_plane_A 7% to 14% more, so a kernel takes what it was measured with.
 template <typename X>
 __device__ __forceinline__ X ld(const void* base, unsigned off)
 {

@@ -89,17 +89,7 @@ __global__ __launch_bounds__(256) void k_scatter(const double2* __restrict__ coe
     const int idx = gindex[e.gidx_off + l];
     double2 c = coef[e.coef_off + l];
     const int dir = e.dir;
-    if (dir == 3) {  // |k+G|^2
-        const int m1 = centered(idx % g.n1, g.n1), m2 = centered((idx / g.n1) % g.n2, g.n2),
-                  m3 = centered(idx / (g.n1 * g.n2), g.n3);
-        double p2 = 0.0;
-        for (int d = 0; d < 3; ++d) {
-            const double p = kcart[3 * e.kidx + d] + g.b[d] * m1 + g.b[3 + d] * m2 + g.b[6 + d] * m3;
-            p2 += p * p;
-        }
-        c.x *= p2;
-        c.y *= p2;
-    } else if (dir >= 0) {
+    if (dir >= 0) {
         const int i1 = idx % g.n1, i2 = (idx / g.n1) % g.n2, i3 = idx / (g.n1 * g.n2);
         const double kg = kcart[3 * e.kidx + dir] + g.b[dir] * centered(i1, g.n1) +
                           g.b[3 + dir] * centered(i2, g.n2) + g.b[6 + dir] * centered(i3, g.n3);

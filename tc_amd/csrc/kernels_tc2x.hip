@@ -244,282 +244,6 @@ __global__ __launch_bounds__(kPencilBlock) void k_tc2x_C(const cpx<T>* __restric
     });
 }
 
-// ================================================================= two-channel form, z-first
-// The two-channel form of kernels_plane_tc2x.hip (bases that do not alias) through the same
-// three z-first passes: records [rho, tau] -> [b, U], orbital sets (phi, L phi) and
-// (phi, L phi, g_d), four accumulators per target.  Used in FP64: 15 grids of traffic per pair
-// instead of 21, half the transforms.
-template <typename T>
-struct Set2 {
-    cpx<T> c, l;
-};
-template <typename T>
-struct Set5 {
-    cpx<T> c, l, g[3];
-};
-
-// (V2 + K^2 u / 2, u) / N per k-q row, y-fastest within each plane: pass B holds one row y per
-// lane when it reads them.
-template <typename T, bool kPoly>
-__global__ __launch_bounds__(256) void k_tc2_table(cpx<T>* __restrict__ table, const double* __restrict__ kqcart,
-                                                   int row0, Geom g, JastrowPair jp, long long N, double invN)
-{
-    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= N) return;
-    const int i2 = (int)(e % g.n2), i1 = (int)((e / g.n2) % g.n1), i3 = (int)(e / ((long long)g.n1 * g.n2));
-    const int m1 = centered(i1, g.n1), m2 = centered(i2, g.n2), m3 = centered(i3, g.n3);
-    const double* kq = kqcart + 3 * (row0 + blockIdx.y);
-    double k2 = 0.0;
-    for (int d = 0; d < 3; ++d) {
-        const double c = kq[d] + g.b[d] * m1 + g.b[3 + d] * m2 + g.b[6 + d] * m3;
-        k2 += c * c;
-    }
-    const double u = jastrow_uk<kPoly>(jp, k2);
-    table[(long long)blockIdx.y * N + e] = cpx<T>{static_cast<T>((jastrow_tc2body<kPoly>(jp, k2) + 0.5 * k2 * u) * invN),
-                                                  static_cast<T>(u * invN)};
-}
-
-template <typename T, int NZ>
-__global__ __launch_bounds__(kPencilBlock, (NZ % 4 == 0 && NZ <= 40 ? 2 : 1)) void k_tc2x2_A(const Set2<T>* __restrict__ app,
-                                                          const Set2<T>* __restrict__ bra,
-                                                          const PairEntry* __restrict__ pairs,
-                                                          cpx<T>* __restrict__ buf, int nxy)
-{
-    constexpr int S = SplitOf<T, NZ>::value;
-    using Split = PencilSplit<S>;
-    constexpr int M = NZ / S;
-    const int h = threadIdx.x / Split::pencils;
-    const int xy0 = blockIdx.x * Split::pencils + (threadIdx.x % Split::pencils);
-    const bool valid = xy0 < nxy;
-    const int xy = valid ? xy0 : 0;
-    const PairEntry pe = pairs[blockIdx.y];
-    const size_t ng = (size_t)nxy * NZ, o = xy + (size_t)h * nxy;  // z = S m + h
-    const Set2<T>* a = app + (size_t)pe.app * ng + o;
-    const Set2<T>* b = bra + (size_t)pe.occ * ng + o;
-    cpx<T>* out = buf + (size_t)blockIdx.y * 2 * ng + xy + (size_t)Split::out_block(h) * M * nxy;  // z = ob*M + k
-    static_for<0, 2>([&](auto cc) {
-        constexpr int c = decltype(cc)::value;
-        cpx<T> v[M];
-        static_for<0, M>([&](auto mc) {
-            constexpr int m = decltype(mc)::value;
-            const Set2<T>*x = a + (size_t)(S * m) * nxy, *w = b + (size_t)(S * m) * nxy;
-            if constexpr (c == 0)
-                v[m] = cmulc(w->c, x->c);
-            else
-                v[m] = cmulc(w->c, x->l) - cmulc(w->l, x->c);
-        });
-        Split::template fft<T, NZ, -1, kSwapF64<T>>(v, h);
-        if (valid) store_pencil_nt<T, M>(v, out + (size_t)c * ng, nxy);
-    });
-}
-
-// P planes z of one pair, both channels: plane slot p, channel c of a lane as in k_tc2x_B with
-// two tiles a plane.  Thread (c = 0, row y) holds rho~ and thread (c = 1, row y) tau~ of the same
-// row; they exchange tau~ and U~ through the tau tile.
-template <typename T, int NP>
-struct Tc2x2Planes {
-    static constexpr int tile_bytes = NP * (NP + 1) * (int)sizeof(cpx<T>);
-    static constexpr int pick()
-    {
-        int best = 1;
-        double best_util = 0.0;
-        for (int p = 1; p <= 8; ++p) {
-            if (2 * p * tile_bytes > kTc2xLdsCap || 2 * p * NP > 512) break;
-            const int lanes = ((2 * p * NP + 63) / 64) * 64;
-            const double util = double(2 * p * NP) / lanes;
-            if (util > best_util + 1e-9) {
-                best_util = util;
-                best = p;
-            }
-        }
-        return best;
-    }
-    static constexpr int planes = pick();
-    static constexpr int threads = ((2 * planes * NP + 63) / 64) * 64;
-};
-
-template <typename T, int NP>
-__global__ __launch_bounds__((Tc2x2Planes<T, NP>::threads)) void k_tc2x2_B(cpx<T>* __restrict__ buf,
-                                                                         const PairEntry* __restrict__ pairs,
-                                                                         const cpx<T>* __restrict__ table, int kq0,
-                                                                         int nz)
-{
-    constexpr int P = Tc2x2Planes<T, NP>::planes;
-    __shared__ PlaneTile<T, NP> S[P * 2];
-    const int pc = threadIdx.x / NP, t = threadIdx.x % NP;
-    const int p = pc >> 1, c = pc & 1;
-    const int z = blockIdx.x * P + p;
-    const bool on = pc < 2 * P && z < nz;
-    const size_t ng = (size_t)NP * NP * nz;
-    PlaneTile<T, NP>& tile = S[on ? pc : 0];
-    cpx<T>* base = buf + ((size_t)blockIdx.y * 2 + (on ? c : 0)) * ng + (size_t)(on ? z : 0) * NP * NP;
-    cpx<T> v[NP];
-    if (on) {
-        load_pencil_nt<T, NP>(v, base + t, NP);  // column x = t
-        fft<T, NP, -1>(v);
-        tile_put_col<T, NP>(tile, v, t);
-    }
-    __syncthreads();
-    if (on) {
-        tile_get_row<T, NP>(tile, v, t);  // row y = t
-        fft<T, NP, -1>(v);
-        if (c == 1) tile_put_row<T, NP>(tile, v, t);
-    }
-    __syncthreads();
-    if (on && c == 0) {
-        PlaneTile<T, NP>& other = S[2 * p + 1];
-        const cpx<T>* w = table + (size_t)(pairs[blockIdx.y].kq - kq0) * ng + (size_t)z * NP * NP + t;
-        static_for<0, NP>([&](auto xc) {
-            constexpr int x = decltype(xc)::value;
-            const cpx<T> s = w[x * NP];
-            const cpx<T> tau = other.a[t][x];
-            other.a[t][x] = scale(v[x], s.im);
-            v[x] = scale(v[x], s.re) + scale(tau, T(0.5) * s.im);
-        });
-    }
-    __syncthreads();
-    if (on) {
-        if (c == 1) tile_get_row<T, NP>(tile, v, t);
-        fft<T, NP, 1>(v);
-        tile_put_row<T, NP>(tile, v, t);
-    }
-    __syncthreads();
-    if (on) {
-        tile_get_col<T, NP>(tile, v, t);
-        fft<T, NP, 1>(v);
-        store_pencil_nt<T, NP>(v, base + t, NP);
-    }
-}
-
-template <typename T, int NZ>
-__global__ __launch_bounds__(kPencilBlock, (NZ % 4 == 0 && NZ <= 40 ? 2 : 1)) void k_tc2x2_C(const cpx<T>* __restrict__ buf,
-                                                          const Set5<T>* __restrict__ ket,
-                                                          const PairEntry* __restrict__ pairs,
-                                                          const TargetEntry* __restrict__ targets,
-                                                          const double* __restrict__ fill, double2* __restrict__ W,
-                                                          float2* __restrict__ Wc, int nxy)
-{
-    constexpr int S = SplitOf<T, NZ>::value;
-    using Split = PencilSplit<S>;
-    constexpr int M = NZ / S;
-    const int h = threadIdx.x / Split::pencils;
-    const int xy0 = blockIdx.x * Split::pencils + (threadIdx.x % Split::pencils);
-    const bool valid = xy0 < nxy;
-    const int xy = valid ? xy0 : 0;
-    const int ob = Split::out_block(h);
-    const TargetEntry te = targets[blockIdx.y];
-    const size_t ng = (size_t)nxy * NZ, o0 = xy + (size_t)ob * M * nxy;
-    double2 acc[4][M];
-    static_for<0, 4 * M>([&](auto ic) {
-        acc[decltype(ic)::value / M][decltype(ic)::value % M] = make_double2(0.0, 0.0);
-    });
-    auto add = [](double2& a, double s, const cpx<T>& x) {
-        a.x += s * static_cast<double>(x.re);
-        a.y += s * static_cast<double>(x.im);
-    };
-#pragma unroll 1
-    for (int pp = te.pair0; pp < te.pair0 + te.npair; ++pp) {
-        const int occ = pairs[pp].occ;
-        const double f = fill[occ];
-        const Set5<T>* q = ket + (size_t)occ * ng + o0;
-        const cpx<T>* in = buf + (size_t)pp * 2 * ng + xy + (size_t)h * nxy;  // z = S m + h
-        cpx<T> v[M];
-        load_pencil<T, M>(v, in + ng, S * nxy);  // U
-        Split::template fft<T, NZ, 1, kSwapF64<T>>(v, h);
-        static_for<0, M>([&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            const Set5<T>* s = q + (size_t)k * nxy;
-            add(acc[0][k], f, v[k] * s->l);
-            static_for<0, 3>([&](auto dc) {
-                constexpr int d = decltype(dc)::value;
-                add(acc[1 + d][k], f, v[k] * s->g[d]);
-            });
-        });
-        __builtin_amdgcn_sched_barrier(0);  // b is loaded when U's registers are free
-        load_pencil<T, M>(v, in, S * nxy);
-        Split::template fft<T, NZ, 1, kSwapF64<T>>(v, h);
-        static_for<0, M>([&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            add(acc[0][k], f, v[k] * q[(size_t)k * nxy].c);
-        });
-    }
-    if (!valid) return;
-    const size_t o = (size_t)te.app * 4 * ng + o0;
-    static_for<0, 4>([&](auto cc) {
-        constexpr int c = decltype(cc)::value;
-        static_for<0, M>([&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            const size_t e = o + (size_t)c * ng + (size_t)k * nxy;
-            add_partial(W + e, Wc + e, acc[c][k].x, acc[c][k].y);
-        });
-    });
-}
-
-void launch_tc2_table(void* table, const double* kqcart, int row0, int nrows, const Geom& g, const JastrowPair& jp,
-                      hipStream_t s)
-{
-    if (nrows == 0) return;
-    const long long N = (long long)g.n1 * g.n2 * g.n3;
-    const dim3 grid((unsigned)((N + 255) / 256), nrows);
-    TCX_POLY_DISPATCH(jp.pdeg > 0, hipLaunchKernelGGL((k_tc2_table<double, kPoly>), grid, dim3(256), 0, s,
-                                                      (cpx<double>*)table, kqcart, row0, g, jp, N, 1.0 / (double)N));
-    TCX_HIP_CHECK(hipGetLastError());
-}
-
-void launch_tc2x2_A(const Geom& g, const void* app, const void* bra, const PairEntry* pairs, int npairs, void* buf,
-                    hipStream_t s)
-{
-    if (npairs == 0) return;
-    if (npairs > 65535) throw Error(TCX_ERR_INTERNAL, "tc2x: too many pairs in one launch");
-    using T = double;
-    const int nxy = g.n1 * g.n2;
-#define TCX_A(NZ)                                                                                            \
-    {                                                                                                        \
-        constexpr int P = 64 / SplitOf<T, NZ>::value;                                                        \
-        hipLaunchKernelGGL((k_tc2x2_A<T, NZ>), dim3((nxy + P - 1) / P, npairs), dim3(kPencilBlock), 0, s,    \
-                           (const Set2<T>*)app, (const Set2<T>*)bra, pairs, (cpx<T>*)buf, nxy);              \
-    }
-    TCX_SIZE_SWITCH(g.n3, TCX_A)
-#undef TCX_A
-    TCX_HIP_CHECK(hipGetLastError());
-}
-
-void launch_tc2x2_B(const Geom& g, void* buf, const PairEntry* pairs, int npairs, const void* table, int kq0,
-                    hipStream_t s)
-{
-    if (npairs == 0) return;
-    if (g.n1 != g.n2) throw Error(TCX_ERR_UNSUPPORTED, "FFT grid must have n1 == n2");
-    using T = double;
-#define TCX_B(NP)                                                                                            \
-    {                                                                                                        \
-        using TP = Tc2x2Planes<T, NP>;                                                                       \
-        hipLaunchKernelGGL((k_tc2x2_B<T, NP>), dim3((g.n3 + TP::planes - 1) / TP::planes, npairs),           \
-                           dim3(TP::threads), 0, s, (cpx<T>*)buf, pairs, (const cpx<T>*)table, kq0, g.n3);   \
-    }
-    TCX_SIZE_SWITCH(g.n1, TCX_B)
-#undef TCX_B
-    TCX_HIP_CHECK(hipGetLastError());
-}
-
-void launch_tc2x2_C(const Geom& g, const void* buf, const void* ket, const PairEntry* pairs, const TargetEntry* targets,
-                    int ntargets, const double* fill, double* W, float* Wc, hipStream_t s)
-{
-    if (ntargets == 0) return;
-    if (ntargets > 65535) throw Error(TCX_ERR_INTERNAL, "tc2x: too many targets in one launch");
-    using T = double;
-    const int nxy = g.n1 * g.n2;
-#define TCX_C(NZ)                                                                                            \
-    {                                                                                                        \
-        constexpr int P = 64 / SplitOf<T, NZ>::value;                                                        \
-        hipLaunchKernelGGL((k_tc2x2_C<T, NZ>), dim3((nxy + P - 1) / P, ntargets), dim3(kPencilBlock), 0, s,  \
-                           (const cpx<T>*)buf, (const Set5<T>*)ket, pairs, targets, fill, (double2*)W,       \
-                           (float2*)Wc, nxy);                                                                \
-    }
-    TCX_SIZE_SWITCH(g.n3, TCX_C)
-#undef TCX_C
-    TCX_HIP_CHECK(hipGetLastError());
-}
-
 // ----------------------------------------------------------------- launchers
 void launch_tc_table(int prec, void* table, const double* kqcart, int row0, int nrows, const Geom& g,
                      const JastrowPair& jp, hipStream_t s)

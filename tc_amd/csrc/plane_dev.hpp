@@ -1,5 +1,5 @@
-// plane_dev.hpp -- device pieces of the plane-first pair pipelines (kernels_plane.hip,
-// kernels_plane_tc2x.hip): the workgroup shape, the column runs and the row loads.
+// plane_dev.hpp -- device pieces of the plane-first pair pipeline (kernels_plane.hip): the
+// workgroup shapes, the column runs and the row loads.
 #pragma once
 
 #include "kernels_common.hpp"
@@ -22,8 +22,8 @@ struct PlaneWg {
 
 // Pass A has no work that tiles share: the fewest wavefronts whose lanes are 84% used, so that
 // a workgroup waits for little but its own transpose.  Against filling the lanes best (FP32, per
-// apply): 36^3 hf2x 4.4 -> 3.9 ms, tc2x 13.0 -> 10.4 ms with 3 planes for 7; 32^3, 30^3 two
-// planes 31 and 1.7 ms against 42 and 2.3 ms with eight.
+// apply): 36^3 4.4 -> 3.9 ms with 3 planes for 7; 32^3, 30^3 two planes 31 and 1.7 ms against 42
+// and 2.3 ms with eight.
 template <typename T, int NP>
 struct PlaneWgA : PlaneWg<T, NP> {
     using B = PlaneWg<T, NP>;
@@ -88,22 +88,6 @@ struct PlaneRuns {
     __device__ __forceinline__ int base(int x) const { return (run[x] >> 16) - (run[x] & 0xff); }
 };
 
-template <typename T, int NZ>
-__device__ __forceinline__ void ld_column(cpx<T> (&v)[NZ], const cpx<T>* base, unsigned off, int cstride)
-{
-    static_for<0, NZ>([&](auto zc) {
-        constexpr int z = decltype(zc)::value;
-        v[z] = ld_nt<T>(base + (size_t)z * cstride, off);
-    });
-}
-template <typename T, int NZ>
-__device__ __forceinline__ void st_column(const cpx<T> (&v)[NZ], cpx<T>* base, unsigned off, int cstride)
-{
-    static_for<0, NZ>([&](auto zc) {
-        constexpr int z = decltype(zc)::value;
-        st_nt<T>(base + (size_t)z * cstride, off, v[z]);
-    });
-}
 // Row t of the record plane at `plane` (uniform) + off (the lane's plane and t), zero outside the
 // support.  The runs are read from memory at every call (the empty asm hides that they do not
 // change): held across a loop they would spill.
@@ -117,17 +101,6 @@ __device__ __forceinline__ void load_row(cpx<T> (&v)[NP], const cpx<T>* plane, u
         constexpr int x = decltype(xc)::value;
         v[x] = cpx<T>{T(0), T(0)};
         if (rr.has(x, t)) v[x] = ld_nt<T>(plane + rr.base(x), off);
-    });
-}
-template <typename T, int NP>
-__device__ __forceinline__ void store_row(const cpx<T> (&v)[NP], cpx<T>* plane, unsigned off,
-                                          const int* __restrict__ runs, int t)
-{
-    asm volatile("" : "+s"(runs));
-    const PlaneRuns<NP> rr(runs);
-    static_for<0, NP>([&](auto xc) {
-        constexpr int x = decltype(xc)::value;
-        if (rr.has(x, t)) st_nt<T>(plane + rr.base(x), off, v[x]);
     });
 }
 

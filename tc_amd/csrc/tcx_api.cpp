@@ -231,9 +231,6 @@ void Context::hermitian_conj()
         std::swap(occR_valid[p], chiR_valid[p]);
         std::swap(d_gradR[p], a_gradR[p]);
         std::swap(gradR_valid[p], a_gradR_valid[p]);
-        std::swap(d_bra[p], a_bra[p]);
-        std::swap(d_ket[p], a_ket[p]);
-        std::swap(sets_valid[p], a_sets_valid[p]);
     }
     std::swap(c_a8, a_a8);
     std::swap(c_hartree, a_hartree);
@@ -254,8 +251,6 @@ void Context::invalidate_states()
     chiR_valid[0] = chiR_valid[1] = false;
     gradR_valid[0] = gradR_valid[1] = false;
     a_gradR_valid[0] = a_gradR_valid[1] = false;
-    sets_valid[0] = sets_valid[1] = false;
-    a_sets_valid[0] = a_sets_valid[1] = false;
     density_valid = false;
     sym_jobs_valid = false;
     plans.clear();
@@ -300,19 +295,13 @@ void Context::set_states(const int* nocc_, const double* filling, const double* 
         TCX_HIP_CHECK(hipMemcpy(d_chi_occ.p, chi_occ, cb, hipMemcpyHostToDevice));
     }
     upload(d_fill, fill.data(), fill.size() * sizeof(double));
-    std::vector<OrbEntry> jobs, gjobs, jobs2, jobs5;
+    std::vector<OrbEntry> jobs, gjobs;
     for (int q = 0; q < nk; ++q)
         for (int i = 0; i < nocc[q]; ++i) {
             const OrbEntry e{occ_coef[q] + (long long)i * npw[q], npw[q], (int)pw_off[q], q, -1};
             jobs.push_back(e);
             for (int d = 0; d < 3; ++d) gjobs.push_back({e.coef_off, e.npw, e.gidx_off, q, d});
-            for (int d : {-1, 3}) jobs2.push_back({e.coef_off, e.npw, e.gidx_off, q, d});
-            for (int d : {-1, 3, 0, 1, 2}) jobs5.push_back({e.coef_off, e.npw, e.gidx_off, q, d});
         }
-    if (method != TCX_METHOD_HF) {
-        upload(d_occ2jobs, jobs2.data(), jobs2.size() * sizeof(OrbEntry));
-        upload(d_occ5jobs, jobs5.data(), jobs5.size() * sizeof(OrbEntry));
-    }
     upload(d_occjobs, jobs.data(), jobs.size() * sizeof(OrbEntry));
     upload(d_occgradjobs, gjobs.data(), gjobs.size() * sizeof(OrbEntry));
     ++states_version;
@@ -519,25 +508,6 @@ void Context::orbitals_to_real(const double* coef, const OrbEntry* d_jobs, int n
     }
 }
 
-// Orbital sets [orbital][N][nc] in precision prec: nc jobs per orbital, FP64 transforms,
-// interleaved and rounded once.
-void Context::orbital_sets(const double* coef, const OrbEntry* d_jobs, int norb, int nc, int prec, void* out)
-{
-    if (norb == 0) return;
-    const size_t g64 = (size_t)N * 16, es = prec == TCX_PREC_FP64 ? 16 : 8;
-    const int chunk = (int)std::max<size_t>(1, std::min<size_t>(norb, ((size_t)1 << 30) / (g64 * nc)));
-    d_tmp64.ensure(g64 * nc * chunk);
-    double* tmp = (double*)d_tmp64.p;
-    for (int c0 = 0; c0 < norb; c0 += chunk) {
-        const int n = std::min(chunk, norb - c0);
-        launch_zero(tmp, g64 * nc * n, stream);
-        launch_scatter(coef, (const int*)d_gindex.p, d_jobs + (size_t)c0 * nc, n * nc, max_npw, tmp, N,
-                       (const double*)d_kcart.p, geo, stream);
-        launch_fft3d(TCX_PREC_FP64, +1, tmp, n * nc, geo, 1.0, stream);
-        launch_interleave(prec, nc, tmp, (char*)out + (size_t)c0 * nc * N * es, n, N, stream);
-    }
-}
-
 void upload(DBuf& buf, const void* src, size_t bytes)
 {
     if (g_capturing)
@@ -611,13 +581,11 @@ void Context::ensure_gradR(int prec)
 // number of pass C groups; targets for four rounds of pass C workgroups over the CUs; both
 // split evenly.  40^3 FP32, 1024 x 1024 orbitals: 94 x 48.  Per apply 96 sources take 20 ms
 // more (pass A reads beyond L2), 32 take 10 ms more and 64 targets 12 ms more (pass C:
-// fewer pairs per update of W; a part-filled last round).  tc2x updates four accumulators per
-// target and takes twice the sources and six rounds: 75 x 48 of 448 x 448 at 40^3, 230 ms
-// against 236 at 75 x 24 (pass A 67 ms, C 101) and 236 at 64 x 96 (84 and 84).
+// fewer pairs per update of W; a part-filled last round).
 // Z-first: enough targets that pass C issues kAutoTargetWaves wavefronts, then as many
 // sources as kAutoBufferGrids pair grids allow (channels = grids per pair record: 1 for
 // hf2x, 4 for tc2x).
-void Context::resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources)
+void Context::resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources) const
 {
     constexpr long kAutoTargetWaves = 8192, kAutoBufferGrids = 8192;
     constexpr long kXcds = 8, kL2Share = 3 << 20, kRounds = 4, kRecordBytes = (long)4 << 30;
@@ -627,15 +595,14 @@ void Context::resolve_shape(int term, int prec, long& tc, long& sc, long ntarget
     const long waves_per_target = ((long)geo.n1 * geo.n2 + 31) / 32;
     tc = (kAutoTargetWaves + waves_per_target - 1) / waves_per_target;
     sc = 0;
-    const bool plane2 = term == 1 && prec == TCX_PREC_FP32 && tc2x_two_channel();
-    if (plane2 || (term == 0 && use_plane_first(prec))) {
-        const long grid_bytes = (long)N * (plane2 ? 16 : 8);  // what pass A reads of a source
-        const PlaneShape ps = plane2 ? plane_tc2x_shape(geo.n1) : plane_shape(geo.n1);
+    if (term == 0 && use_plane_first(prec)) {
+        const long grid_bytes = (long)N * 8;
+        const PlaneShape ps = plane_shape(geo.n1);
         auto even = [](long n, long most) { return (n + (n + most - 1) / most - 1) / ((n + most - 1) / most); };
         auto whole = [&](long n) { return std::max<long>(1, n / ps.group) * ps.group; };
-        const long most = whole((plane2 ? 2 : 1) * kXcds * kL2Share / grid_bytes);
+        const long most = whole(kXcds * kL2Share / grid_bytes);
         sc = std::min(most, whole(even(nsources, most) + ps.group - 1));
-        tc = std::max<long>(1, (plane2 ? 6 : kRounds) * ps.slots / geo.n3);
+        tc = std::max<long>(1, kRounds * ps.slots / geo.n3);
         tc = even(ntargets, std::max<long>(1, std::min(tc, kRecordBytes / (sc * grid_bytes))));
     }
     if (shape_targets[term] > 0) tc = shape_targets[term];
@@ -731,14 +698,13 @@ const BandJobs& Context::get_band_jobs(const std::vector<int>& nb)
     }
     J.n_app = (int)J.app_first[nk];
     // one scatter/gather job and one divergence job per applied band, in band order
-    std::vector<OrbEntry> appjobs, appgradjobs, app2jobs;
+    std::vector<OrbEntry> appjobs, appgradjobs;
     std::vector<DivEntry> divjobs;
     for (int k = 0; k < nk; ++k)
         for (int j = 0; j < nb[k]; ++j) {
             const OrbEntry e{J.app_coef[k] + (long long)j * npw[k], npw[k], (int)pw_off[k], k, -1};
             appjobs.push_back(e);
             for (int d = 0; d < 3; ++d) appgradjobs.push_back({e.coef_off, e.npw, e.gidx_off, k, d});
-            for (int d : {-1, 3}) app2jobs.push_back({e.coef_off, e.npw, e.gidx_off, k, d});
             if (zw_set && zw_k[k])  // the states given for a zero-weight k
                 divjobs.push_back({e.coef_off, zw_coef[k], npw[k], zw_n[k], zw_first[k], k});
             else
@@ -746,7 +712,6 @@ const BandJobs& Context::get_band_jobs(const std::vector<int>& nb)
         }
     upload_tables(J.tables, {{&J.d_appjobs, appjobs.data(), appjobs.size() * sizeof(OrbEntry)},
                              {&J.d_appgradjobs, appgradjobs.data(), appgradjobs.size() * sizeof(OrbEntry)},
-                             {&J.d_app2jobs, app2jobs.data(), app2jobs.size() * sizeof(OrbEntry)},
                              {&J.d_divjobs, divjobs.data(), divjobs.size() * sizeof(DivEntry)}});
     return band_jobs.emplace(nb, std::move(J)).first->second;
 }

@@ -82,7 +82,7 @@ struct OrbEntry {
     int npw;
     int gidx_off;         // offset into the concatenated gindex array
     int kidx;             // k-point (for gradients)
-    int dir;              // -1: plain scatter; 0..2: multiply by the Cartesian (k+G)_dir; 3: by |k+G|^2
+    int dir;              // -1: plain scatter; 0..2: multiply by the Cartesian (k+G)_dir
 };
 
 // Divergence-correction job for one applied band (k, j).
@@ -145,30 +145,6 @@ void launch_plane_Z(const Geom& g, void* rec, const PairEntry* pairs, int npairs
 void launch_plane_C(const Geom& g, const void* rec, const void* occ, const PairEntry* pairs,
                     const TargetEntry* targets, int ntargets, const PlaneCols& pc, const double* fill, double* W,
                     float* Wc, hipStream_t s);
-// two-channel tc2x (kernels_plane_tc2x.hip): orbital sets [orbital][N][nc] (nc = 2: phi, L phi; 5: phi, L phi,
-// g_d), the passes and the gather of the four accumulators
-void launch_interleave(int prec, int nc, const double* in, void* out, int norb, long long N, hipStream_t s);
-void launch_gather_tc2x(const double* W, const int* gindex, const OrbEntry* jobs, int njobs, int max_npw, double* out,
-                        long long N, const double* kcart, const Geom& g, double factor, hipStream_t s);
-// z-first, FP64
-void launch_tc2_table(void* table, const double* kqcart, int row0, int nrows, const Geom& g, const JastrowPair& jp,
-                      hipStream_t s);
-void launch_tc2x2_A(const Geom& g, const void* app, const void* bra, const PairEntry* pairs, int npairs, void* buf,
-                    hipStream_t s);
-void launch_tc2x2_B(const Geom& g, void* buf, const PairEntry* pairs, int npairs, const void* table, int kq0,
-                    hipStream_t s);
-void launch_tc2x2_C(const Geom& g, const void* buf, const void* ket, const PairEntry* pairs, const TargetEntry* targets,
-                    int ntargets, const double* fill, double* W, float* Wc, hipStream_t s);
-PlaneShape plane_tc2x_shape(int n1);
-void launch_plane_tc_table(void* tab, const double* kqcart, int row0, int nrows, const PlaneCols& pc, const Geom& g,
-                           const JastrowPair& jp, hipStream_t s);
-void launch_plane_tc2x_A(const Geom& g, const void* app, const void* bra, const PairEntry* pairs, int ntargets,
-                         int nsrc, const PlaneCols& pc, void* rec, hipStream_t s);
-void launch_plane_tc2x_Z(const Geom& g, void* rec, const PairEntry* pairs, int npairs, const void* tab, int kq0,
-                         const PlaneCols& pc, hipStream_t s);
-void launch_plane_tc2x_C(const Geom& g, const void* rec, const void* ket, const PairEntry* pairs,
-                         const TargetEntry* targets, int ntargets, const PlaneCols& pc, const double* fill, double* W,
-                         float* Wc, hipStream_t s);
 void launch_hf2x_A(int prec, const Geom& g, const void* phiR_app, const void* phiR_occ, const PairEntry* pairs,
                    int npairs, void* buf, hipStream_t s);
 void launch_coulomb_table(int prec, void* table, const double* kqcart, int row0, int nrows, const Geom& g,

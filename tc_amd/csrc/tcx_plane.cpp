@@ -1,4 +1,4 @@
-// tcx_plane.cpp -- host side of the plane-first pair pipelines (kernels_plane.hip): the
+// tcx_plane.cpp -- host side of the plane-first pair pipeline (kernels_plane.hip): the
 // support columns of the basis and the hf2x launch sequence.
 //
 // The pair density of (k,j | q,i) has G-space components G = G_k - G_q with G_k in the
@@ -88,7 +88,7 @@ const PlaneCols& Context::plane_cols()
     // record rows start on 128-byte lines, unless that would make them longer than a grid plane
     cols.pc.cstride = std::min((cols.pc.ncol + 15) / 16 * 16, n1 * n2);
     cols.pc.rot = posmod(first_ky, n2);
-    // no sum or difference of three basis vectors that matters wraps (tc2x_two_channel)
+    // every basis inside a span s of Miller indices per direction with 2 s < n (basis_no_alias)
     int mn[3] = {none_lo, none_lo, none_lo}, mx[3] = {none_hi, none_hi, none_hi};
     const int n[3] = {geo.n1, geo.n2, geo.n3};
     for (const int e : gindex_h) {
@@ -133,58 +133,13 @@ void Context::hf2x_plane_first(const Plan& P)
     }
 }
 
-// The two-channel form of tc2x replaces K.p and K.p'' of a pair's plane waves by their squares
-// and P.p'', which needs the FFT grid to hold K = p - p' itself (every difference within the
-// centred range (-n/2, n/2]) and P = K + p'' not to be reached by a wrapped sum: with all bases
-// inside a span s of Miller indices per direction, 2 s < n implies both.  Bases that alias keep
-// the four-channel form, whose products and gradients the wrapped indices enter as in the
-// reference.
-bool Context::tc2x_two_channel()
+// No difference of two basis vectors reaches the Nyquist index or wraps: with every basis inside a
+// span s of Miller indices per direction, 2 s < n keeps the differences inside (-n/2, n/2), where
+// -G has the index opposite to G's and K(-G) = -K(G).
+bool Context::basis_no_alias()
 {
     plane_cols();
     return cols.no_alias;
-}
-
-void Context::ensure_tc2x_sets(int prec)
-{
-    if (sets_valid[prec]) return;
-    const size_t es = prec == TCX_PREC_FP64 ? 16 : 8;
-    const double* right = (const double*)d_phi_occ.p;
-    const double* left = method == TCX_METHOD_BITC ? (const double*)d_chi_occ.p : right;
-    d_bra[prec].ensure(std::max<size_t>((size_t)n_occ * 2 * N * es, 16));
-    d_ket[prec].ensure(std::max<size_t>((size_t)n_occ * 5 * N * es, 16));
-    orbital_sets(left, (const OrbEntry*)d_occ2jobs.p, n_occ, 2, prec, d_bra[prec].p);
-    orbital_sets(right, (const OrbEntry*)d_occ5jobs.p, n_occ, 5, prec, d_ket[prec].p);
-    sets_valid[prec] = true;
-}
-
-// The plane-first passes of the two-channel form (FP32-split) into the four accumulators of
-// every applied band; W was cleared by the caller and d_appR holds the applied bands' sets.
-void Context::tc2x_plane_first(const Plan& P)
-{
-    const PlaneCols& pc = plane_cols();
-    const size_t plane = (size_t)geo.n3 * pc.cstride;
-    d_pairbuf.ensure((size_t)std::max(1, P.max_launch_pairs) * 2 * plane * 8);
-    int max_rows = 1;
-    for (const Launch& L : P.launches) max_rows = std::max(max_rows, L.nkq);
-    d_ktab.ensure((size_t)max_rows * plane * 8);
-    for (const Launch& L : P.launches) {
-        const PairEntry* pairs = (const PairEntry*)P.d_pairs.p + L.pair0;
-        const TargetEntry* targets = (const TargetEntry*)P.d_targets.p + L.target0;
-        launch_plane_tc_table(d_ktab.p, (const double*)P.d_kq.p, L.kq0, L.nkq, pc, geo, jastrow_pair(L.spin, L.spin),
-                              stream);  // tc2x.cpp:269-271 (ispin, ispin)
-        timed(0, L.npairs, [&] {
-            launch_plane_tc2x_A(geo, d_appR.p, d_bra[TCX_PREC_FP32].p, pairs, L.ntargets, L.npairs / L.ntargets, pc,
-                                d_pairbuf.p, stream);  // every source of a launch pairs with every target
-        });
-        timed(1, L.npairs, [&] {
-            launch_plane_tc2x_Z(geo, d_pairbuf.p, pairs, L.npairs, d_ktab.p, L.kq0, pc, stream);
-        });
-        timed(2, L.npairs, [&] {
-            launch_plane_tc2x_C(geo, d_pairbuf.p, d_ket[TCX_PREC_FP32].p, pairs, targets, L.ntargets, pc,
-                                (const double*)d_fill.p, (double*)d_W.p, (float*)d_Wc.p, stream);
-        });
-    }
 }
 
 }  // namespace tcx

@@ -17,63 +17,43 @@ void Context::tc2x(const int* nb_, const double* phi, double* out, int prec, uns
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     if (P.n_app > 0) {
         const bool bitc = method == TCX_METHOD_BITC;
+        ensure_occR(prec);
+        ensure_gradR(prec);
+        if (bitc) ensure_chiR(prec);
+        const void* chiR = bitc ? d_chiR[prec].p : d_occR[prec].p;  // bra orbital (tc2x.cpp:306)
+        const size_t es = prec == TCX_PREC_FP64 ? 16 : 8;
+        d_appR.ensure((size_t)P.n_app * N * es);
+        d_appGrad.ensure((size_t)3 * P.n_app * N * es);
+        timed(3, 0, [&] {
+            orbitals_to_real(io.phi, (const OrbEntry*)P.d_appjobs.p, P.n_app, prec, d_appR.p);
+            orbitals_to_real(io.phi, (const OrbEntry*)P.d_appgradjobs.p, 3 * P.n_app, prec, d_appGrad.p);
+        });
+        begin_W(P.n_app);
+        d_pairbuf.ensure((size_t)std::max(1, P.max_launch_pairs) * 4 * N * es);
+        int max_rows = 1;
+        for (const Launch& L : P.launches) max_rows = std::max(max_rows, L.nkq);
+        d_ktab.ensure((size_t)max_rows * N * es);
+        for (const Launch& L : P.launches) {
+            const PairEntry* pairs = (const PairEntry*)P.d_pairs.p + L.pair0;
+            const TargetEntry* targets = (const TargetEntry*)P.d_targets.p + L.target0;
+            const JastrowPair jp = jastrow_pair(L.spin, L.spin);  // tc2x.cpp:269-271 (ispin, ispin)
+            launch_tc_table(prec, d_ktab.p, (const double*)P.d_kq.p, L.kq0, L.nkq, geo, jp, stream);
+            timed(0, L.npairs, [&] {
+                launch_tc2x_A(prec, geo, d_appR.p, d_appGrad.p, chiR, pairs, L.npairs, d_pairbuf.p, stream);
+            });
+            timed(1, L.npairs, [&] {
+                launch_tc2x_B(prec, geo, d_pairbuf.p, pairs, L.npairs, d_ktab.p, L.kq0, (const double*)P.d_kq.p,
+                              stream);
+            });
+            timed(2, L.npairs, [&] {
+                launch_tc2x_C(prec, geo, d_pairbuf.p, d_occR[prec].p, d_gradR[prec].p, pairs, targets, L.ntargets,
+                              (const double*)d_fill.p, (double*)d_W.p, (float*)d_Wc.p, stream);
+            });
+        }
         // two_body_factor, src/calc_hamiltonian_tc2x.cpp:32-33
         double factor = -1.0 / (num_kpoints * volume);
         if (nspin == 1) factor /= 2.0;
-        if (tc2x_two_channel()) {
-            const size_t es = prec == TCX_PREC_FP64 ? 16 : 8;
-            ensure_tc2x_sets(prec);
-            d_appR.ensure((size_t)2 * P.n_app * N * es);
-            timed(3, 0, [&] {
-                orbital_sets(io.phi, (const OrbEntry*)P.d_app2jobs.p, P.n_app, 2, prec, d_appR.p);
-            });
-            begin_W(4 * P.n_app);
-            if (prec == TCX_PREC_FP32)
-                tc2x_plane_first(P);
-            else
-                tc2x_two_channel_z(P);
-            launch_add_into((double*)d_W.p, (const float*)d_Wc.p, (long long)4 * P.n_app * N, stream);
-            timed(3, 0, [&] {
-                launch_fft3d(TCX_PREC_FP64, -1, d_W.p, 4 * P.n_app, geo, 1.0 / (double)N, stream);
-            });
-            launch_gather_tc2x((const double*)d_W.p, (const int*)d_gindex.p, (const OrbEntry*)P.d_appjobs.p, P.n_app,
-                               max_npw, io.out, N, (const double*)d_kcart.p, geo, factor, stream);
-        } else {
-            ensure_occR(prec);
-            ensure_gradR(prec);
-            if (bitc) ensure_chiR(prec);
-            const void* chiR = bitc ? d_chiR[prec].p : d_occR[prec].p;  // bra orbital (tc2x.cpp:306)
-            const size_t es = prec == TCX_PREC_FP64 ? 16 : 8;
-            d_appR.ensure((size_t)P.n_app * N * es);
-            d_appGrad.ensure((size_t)3 * P.n_app * N * es);
-            timed(3, 0, [&] {
-                orbitals_to_real(io.phi, (const OrbEntry*)P.d_appjobs.p, P.n_app, prec, d_appR.p);
-                orbitals_to_real(io.phi, (const OrbEntry*)P.d_appgradjobs.p, 3 * P.n_app, prec, d_appGrad.p);
-            });
-            begin_W(P.n_app);
-            d_pairbuf.ensure((size_t)std::max(1, P.max_launch_pairs) * 4 * N * es);
-            int max_rows = 1;
-            for (const Launch& L : P.launches) max_rows = std::max(max_rows, L.nkq);
-            d_ktab.ensure((size_t)max_rows * N * es);
-            for (const Launch& L : P.launches) {
-                const PairEntry* pairs = (const PairEntry*)P.d_pairs.p + L.pair0;
-                const TargetEntry* targets = (const TargetEntry*)P.d_targets.p + L.target0;
-                const JastrowPair jp = jastrow_pair(L.spin, L.spin);  // tc2x.cpp:269-271 (ispin, ispin)
-                launch_tc_table(prec, d_ktab.p, (const double*)P.d_kq.p, L.kq0, L.nkq, geo, jp, stream);
-                timed(0, L.npairs, [&] {
-                    launch_tc2x_A(prec, geo, d_appR.p, d_appGrad.p, chiR, pairs, L.npairs, d_pairbuf.p, stream);
-                });
-                timed(1, L.npairs, [&] {
-                    launch_tc2x_B(prec, geo, d_pairbuf.p, pairs, L.npairs, d_ktab.p, L.kq0, (const double*)P.d_kq.p,
-                                  stream);
-                });
-                timed(2, L.npairs, [&] {
-                    launch_tc2x_C(prec, geo, d_pairbuf.p, d_occR[prec].p, d_gradR[prec].p, pairs, targets, L.ntargets,
-                                  (const double*)d_fill.p, (double*)d_W.p, (float*)d_Wc.p, stream);
-                });
-            }
-            finish_W(P, io, factor);
-        }
+        finish_W(P, io, factor);
         std::vector<double> kv;
         tc2x_kvaux(kv);
         if (div_enabled && std::any_of(kv.begin(), kv.end(), [](double x) { return x != 0.0; })) {
@@ -88,29 +68,6 @@ void Context::tc2x(const int* nb_, const double* phi, double* out, int prec, uns
         }
     }
     end_apply(io);
-}
-
-// The z-first passes of the two-channel form (FP64) into the four accumulators of every
-// applied band.
-void Context::tc2x_two_channel_z(const Plan& P)
-{
-    d_pairbuf.ensure((size_t)std::max(1, P.max_launch_pairs) * 2 * N * 16);
-    int max_rows = 1;
-    for (const Launch& L : P.launches) max_rows = std::max(max_rows, L.nkq);
-    d_ktab.ensure((size_t)max_rows * N * 16);
-    for (const Launch& L : P.launches) {
-        const PairEntry* pairs = (const PairEntry*)P.d_pairs.p + L.pair0;
-        const TargetEntry* targets = (const TargetEntry*)P.d_targets.p + L.target0;
-        launch_tc2_table(d_ktab.p, (const double*)P.d_kq.p, L.kq0, L.nkq, geo, jastrow_pair(L.spin, L.spin), stream);
-        timed(0, L.npairs, [&] {
-            launch_tc2x2_A(geo, d_appR.p, d_bra[TCX_PREC_FP64].p, pairs, L.npairs, d_pairbuf.p, stream);
-        });
-        timed(1, L.npairs, [&] { launch_tc2x2_B(geo, d_pairbuf.p, pairs, L.npairs, d_ktab.p, L.kq0, stream); });
-        timed(2, L.npairs, [&] {
-            launch_tc2x2_C(geo, d_pairbuf.p, d_ket[TCX_PREC_FP64].p, pairs, targets, L.ntargets,
-                           (const double*)d_fill.p, (double*)d_W.p, (float*)d_Wc.p, stream);
-        });
-    }
 }
 
 void Context::ensure_density()

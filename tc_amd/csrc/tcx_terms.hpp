@@ -110,7 +110,6 @@ struct BandJobs {
     int n_app = 0;
     DView d_appjobs;      // OrbEntry per applied band (band order)
     DView d_appgradjobs;  // three OrbEntry (dir 0..2) per applied band
-    DView d_app2jobs;     // two OrbEntry (phi, |k+G|^2 phi) per applied band
     DView d_divjobs;      // DivEntry per applied band
 };
 struct BandJobSet : BandJobs {
@@ -203,16 +202,8 @@ struct Context {
         DBuf buf;
     } cols;
     const PlaneCols& plane_cols();
+    bool basis_no_alias();
     void hf2x_plane_first(const Plan& P);
-    // the two-channel form of tc2x (kernels_plane_tc2x.hip) and its orbital sets per precision
-    bool tc2x_two_channel();
-    void ensure_tc2x_sets(int prec);
-    void orbital_sets(const double* coef, const OrbEntry* d_jobs, int norb, int nc, int prec, void* out);
-    void tc2x_plane_first(const Plan& P);
-    void tc2x_two_channel_z(const Plan& P);
-    DBuf d_bra[2], d_ket[2], a_bra[2], a_ket[2];  // a_: of the other orientation (hermitian_conj)
-    bool sets_valid[2] = {false, false}, a_sets_valid[2] = {false, false};
-    DBuf d_occ2jobs, d_occ5jobs;  // OrbEntry (phi, L) and (phi, L, g_d) per occupied orbital
     std::map<std::tuple<std::vector<int>, long, long>, Plan> plans;
     std::map<std::vector<int>, BandJobSet> band_jobs;  // cleared with the plans that view them
     const BandJobs& get_band_jobs(const std::vector<int>& nb);
@@ -340,7 +331,7 @@ struct Context {
     void jastrow_kernels(int s1, int s2, long long n, const double* G2, double* uk, double* v);
     void ensure_density();
 
-    void resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources);
+    void resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources) const;
     static constexpr int kPlanJobs = -1;
     const Plan& get_plan(const std::vector<int>& nb, int term, int prec = 0);
     void check_apply_args(const int* nb, const double* phi, const double* out, int prec);
