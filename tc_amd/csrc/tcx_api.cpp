@@ -198,12 +198,21 @@ void Context::set_basis(const int* npw_, const int* gindex)
         off[k + 1] = off[k] + n_[k];
     }
     const long long nphys = off[nk_phys];
-    for (long long l = 0; l < nphys; ++l)
+    std::vector<unsigned char> seen((size_t)N, 0);  // grid points that some basis holds
+    for (long long l = 0; l < nphys; ++l) {
         require(gindex[l] >= 0 && gindex[l] < N, TCX_ERR_ARG, "set_basis: gindex outside the FFT grid");
+        seen[gindex[l]] = 1;
+    }
     std::vector<int> gi;
     for (int s = 0; s < nspin; ++s) gi.insert(gi.end(), gindex, gindex + nphys);
+    const size_t ng = gi.size();
+    const std::vector<int> columns = set_columns(seen);
+    gi.insert(gi.end(), columns.begin(), columns.end());
     d_gindex.ensure(gi.size() * sizeof(int));
     TCX_HIP_CHECK(hipMemcpy(d_gindex.p, gi.data(), gi.size() * sizeof(int), hipMemcpyHostToDevice));
+    cols.run = (const int*)d_gindex.p + ng;
+    cols.colxy = cols.run + geo.n1;
+    gi.resize(ng);
     npw = std::move(n_);
     pw_off = std::move(off);
     max_npw = *std::max_element(npw.begin(), npw.end());
@@ -244,7 +253,6 @@ void Context::hermitian_conj()
 
 void Context::invalidate_states()
 {
-    if (!basis_set) cols.valid = false;
     clear_zero_weight();  // its states live in the orbital arrays that a setter replaces
     invalidate_local();
     occR_valid[0] = occR_valid[1] = false;

@@ -232,14 +232,13 @@ void Context::hf2x_noalloc(const int* nb_, const double* phi, double* out, int p
         for (const L& l : launches) {
             const PairEntry* lp = d_pairs + l.pair0;
             const TargetEntry* lt = d_targets + l.target0;
-            // the pass order of tcx_hf2x, whose FP32 call before this one built the columns; a
-            // plane-first record is no larger than a grid
-            if (use_plane_first(prec) && cols.valid) {
-                launch_plane_coulomb(ktab, d_kq, l.kq0, l.nkq, cols.pc, geo, stream);
-                launch_plane_A(geo, appR, d_occR[prec].p, lp, l.ntargets, l.npairs / l.ntargets, cols.pc, pairbuf,
+            // the pass order of tcx_hf2x; a plane-first record is no larger than a grid
+            if (use_plane_first(prec)) {
+                launch_plane_coulomb(ktab, d_kq, l.kq0, l.nkq, cols, geo, stream);
+                launch_plane_A(geo, appR, d_occR[prec].p, lp, l.ntargets, l.npairs / l.ntargets, cols, pairbuf,
                                stream);
-                launch_plane_Z(geo, pairbuf, lp, l.npairs, ktab, l.kq0, cols.pc, stream);
-                launch_plane_C(geo, pairbuf, d_occR[prec].p, lp, lt, l.ntargets, cols.pc, (const double*)d_fill.p, W,
+                launch_plane_Z(geo, pairbuf, lp, l.npairs, ktab, l.kq0, cols, stream);
+                launch_plane_C(geo, pairbuf, d_occR[prec].p, lp, lt, l.ntargets, cols, (const double*)d_fill.p, W,
                                nullptr, stream);
                 continue;
             }

@@ -38,18 +38,39 @@ bool Context::use_plane_first(int prec) const
 // With the ky span of the whole set at most n2, ky rotated by the smallest difference makes
 // every run contiguous; a run that still wraps (bases that alias on the grid) takes every ky.
 // Hulls and the union only add columns, so the record holds every non-zero one.
-const PlaneCols& Context::plane_cols()
+// Found by tcx_set_basis from the grid points that some basis holds (`seen`): one pass over the
+// grid without a division per plane wave.  Returns run[n1] and colxy[ncol]; they go to the device
+// behind the grid indices, in the same copy.
+std::vector<int> Context::set_columns(const std::vector<unsigned char>& seen)
 {
-    if (cols.valid) return cols.pc;
-    const int n1 = geo.n1, n2 = geo.n2;
-    // per centred kx: [lo, hi] of centred ky over all bases (lo > hi: none)
+    const int n1 = geo.n1, n2 = geo.n2, n3 = geo.n3, nxy = n1 * n2;
     const int none_lo = 1 << 20, none_hi = -(1 << 20);
-    std::vector<int> lo(n1, none_lo), hi(n1, none_hi);
-    for (const int e : gindex_h) {
-        const int i1 = e % n1, m2 = centered_host((e / n1) % n2, n2);
-        lo[i1] = std::min(lo[i1], m2);
-        hi[i1] = std::max(hi[i1], m2);
+    std::vector<unsigned char> col(nxy, 0);
+    int mn[3] = {none_lo, none_lo, none_lo}, mx[3] = {none_hi, none_hi, none_hi};  // centred indices held
+    auto widen = [&](int d, int m) {
+        mn[d] = std::min(mn[d], m);
+        mx[d] = std::max(mx[d], m);
+    };
+    for (int i3 = 0; i3 < n3; ++i3) {
+        const unsigned char* p = seen.data() + (size_t)i3 * nxy;
+        unsigned char any = 0;
+        for (int e = 0; e < nxy; ++e) {
+            col[e] |= p[e];
+            any |= p[e];
+        }
+        if (any) widen(2, centered_host(i3, n3));
     }
+    // per kx: [lo, hi] of centred ky over all bases (lo > hi: none)
+    std::vector<int> lo(n1, none_lo), hi(n1, none_hi);
+    for (int i2 = 0; i2 < n2; ++i2)
+        for (int i1 = 0; i1 < n1; ++i1) {
+            if (!col[(size_t)i2 * n1 + i1]) continue;
+            const int m2 = centered_host(i2, n2);
+            widen(0, centered_host(i1, n1));
+            widen(1, m2);
+            lo[i1] = std::min(lo[i1], m2);
+            hi[i1] = std::max(hi[i1], m2);
+        }
     std::vector<int> dlo(n1, none_lo), dhi(n1, none_hi);
     for (int a = 0; a < n1; ++a) {
         if (lo[a] > hi[a]) continue;
@@ -80,35 +101,24 @@ const PlaneCols& Context::plane_cols()
         run[x] = l | (len << 8) | ((int)colxy.size() << 16);
         for (int j = 0; j < len; ++j) colxy.push_back(x | (posmod(first_ky + l + j, n2) << 16));
     }
-    cols.pc.ncol = (int)colxy.size();
-    run.insert(run.end(), colxy.begin(), colxy.end());
-    upload(cols.buf, run.data(), run.size() * sizeof(int));
-    cols.pc.run = (const int*)cols.buf.p;
-    cols.pc.colxy = cols.pc.run + n1;
+    cols.ncol = (int)colxy.size();
     // record rows start on 128-byte lines, unless that would make them longer than a grid plane
-    cols.pc.cstride = std::min((cols.pc.ncol + 15) / 16 * 16, n1 * n2);
-    cols.pc.rot = posmod(first_ky, n2);
-    // every basis inside a span s of Miller indices per direction with 2 s < n (basis_no_alias)
-    int mn[3] = {none_lo, none_lo, none_lo}, mx[3] = {none_hi, none_hi, none_hi};
-    const int n[3] = {geo.n1, geo.n2, geo.n3};
-    for (const int e : gindex_h) {
-        const int m[3] = {centered_host(e % n1, n1), centered_host((e / n1) % n2, n2),
-                          centered_host(e / (n1 * n2), geo.n3)};
-        for (int d = 0; d < 3; ++d) {
-            mn[d] = std::min(mn[d], m[d]);
-            mx[d] = std::max(mx[d], m[d]);
-        }
-    }
-    cols.no_alias = true;
-    for (int d = 0; d < 3; ++d) cols.no_alias = cols.no_alias && 2 * (mx[d] - mn[d]) < n[d];
-    cols.valid = true;
-    return cols.pc;
+    cols.cstride = std::min((cols.ncol + 15) / 16 * 16, nxy);
+    cols.rot = posmod(first_ky, n2);
+    // No difference of two basis vectors reaches the Nyquist index or wraps: with every basis inside a
+    // span s of Miller indices per direction, 2 s < n keeps the differences inside (-n/2, n/2), where
+    // -G has the index opposite to G's and K(-G) = -K(G).
+    const int n[3] = {n1, n2, n3};
+    basis_no_alias = true;
+    for (int d = 0; d < 3; ++d) basis_no_alias = basis_no_alias && 2 * (mx[d] - mn[d]) < n[d];
+    run.insert(run.end(), colxy.begin(), colxy.end());
+    return run;
 }
 
 // The three plane-first passes of every launch; W (FP64) was cleared by the caller.
 void Context::hf2x_plane_first(const Plan& P)
 {
-    const PlaneCols& pc = plane_cols();
+    const PlaneCols& pc = cols;
     hf2x_record_cols = pc.ncol;
     const size_t es = 8, plane = (size_t)geo.n3 * pc.cstride;
     d_pairbuf.ensure((size_t)std::max(1, P.max_launch_pairs) * plane * es);
@@ -131,15 +141,6 @@ void Context::hf2x_plane_first(const Plan& P)
                            (const double*)d_fill.p, (double*)d_W.p, (float*)d_Wc.p, stream);
         });
     }
-}
-
-// No difference of two basis vectors reaches the Nyquist index or wraps: with every basis inside a
-// span s of Miller indices per direction, 2 s < n keeps the differences inside (-n/2, n/2), where
-// -G has the index opposite to G's and K(-G) = -K(G).
-bool Context::basis_no_alias()
-{
-    plane_cols();
-    return cols.no_alias;
 }
 
 }  // namespace tcx

@@ -66,7 +66,7 @@ const PairSet& Context::pair_set(const std::vector<int>& nb, PairKind kind, int 
 // 40^3 FP32 BITC, 2x2x2 k, 12 bands: products and xy passes of the phase 20.7 -> 10.2 ms.
 const PairSet& Context::q_pair_set(int nin, int prec)
 {
-    const bool half = !sym_set && basis_no_alias();
+    const bool half = !sym_set && basis_no_alias;
     auto key = std::make_tuple(std::vector<int>(), kPairsQ * 1000 + 2 * nin + prec);
     auto it = pairsets.find(key);
     if (it != pairsets.end()) return it->second;

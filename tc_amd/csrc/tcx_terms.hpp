@@ -195,14 +195,11 @@ struct Context {
     double hf2x_record_cols = 0;  // (kx, ky) columns per plane of the last hf2x apply's records
     bool in_davidson = false;     // an apply of tcx_davidson runs (use_plane_first)
     bool use_plane_first(int prec) const;
-    // support columns of the pair records, from the basis (dropped by tcx_set_basis and what precedes it)
-    struct {
-        bool valid = false, no_alias = false;
-        PlaneCols pc{};
-        DBuf buf;
-    } cols;
-    const PlaneCols& plane_cols();
-    bool basis_no_alias();
+    // support columns of the pair records and whether differences of basis vectors stay inside the
+    // grid; both belong to the basis (tcx_set_basis), their tables lie behind d_gindex's indices
+    PlaneCols cols{};
+    bool basis_no_alias = false;
+    std::vector<int> set_columns(const std::vector<unsigned char>& seen);
     void hf2x_plane_first(const Plan& P);
     std::map<std::tuple<std::vector<int>, long, long>, Plan> plans;
     std::map<std::vector<int>, BandJobSet> band_jobs;  // cleared with the plans that view them

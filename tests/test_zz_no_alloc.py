@@ -67,3 +67,34 @@ def test_hf2x_noalloc_matches_hf2x(prec):
         for b in bufs:
             b.free()
         eng.close()
+
+
+def test_hf2x_noalloc_takes_the_order_of_hf2x():
+    """The pass order follows from the precision and tcx_set_pipeline_order alone, not from which
+    call put the occupied orbitals in real space: after an FP32 Davidson (whose own applies run
+    z-first) the result is that of a later call after tcx_hf2x, bit for bit."""
+    sys_ = S.tiny_system(method="HF", n=(16, 16, 16), kmesh=(2, 1, 1), nbands=3, nocc=3, seed_stream=84)
+    eng = tcx.Engine(0)
+    bufs = []
+    try:
+        nb, phi = S.applied_bands(sys_, nb=np.array([3, 2], np.int32), seed=85)
+        got = {}
+        for first in ("davidson", "hf2x"):
+            eng.load_system(sys_)
+            d_in = eng.to_device(phi)
+            d_out = eng.device_buffer(phi.nbytes)
+            bufs += [d_in, d_out]
+            if first == "davidson":
+                eng.davidson(nb, phi, np.zeros(int(nb.sum()), complex), precision=tcx.PREC_FP32)
+            else:
+                eng._term_device("hf2x", nb, d_in.ptr, d_out.ptr, tcx.PREC_FP32)
+            d_out.zero()
+            st = _noalloc(eng, nb, d_in.ptr, d_out.ptr, tcx.PREC_FP32)
+            assert st == tcx.TCX_OK, eng.L.tcx_last_error(eng.h)
+            got[first] = d_out.download(np.complex128)
+        assert np.abs(got["hf2x"]).max() > 0
+        assert np.array_equal(got["davidson"], got["hf2x"])
+    finally:
+        for b in bufs:
+            b.free()
+        eng.close()
