@@ -4,6 +4,8 @@ Tolerances (written here, per result):
   FP64 path : max |delta| <= 1e-10 * max |ref|  (FFT round-off only)
   FP32 path : per band ||delta||/||ref|| <= 2e-5 and |delta E_x| <= 1e-6 Ha/cell
 """
+import math
+
 import numpy as np
 import pytest
 
@@ -18,6 +20,13 @@ from test_oracle import plane_wave_system
 pytestmark = pytest.mark.gpu
 
 HF_GOLDEN = [n for n in golden_names() if n.startswith("hf_")]
+
+
+def fp32_rounding(n, transforms=2):
+    """Bound on the FP32-split error of a band: about 2 log2 N roundings of 2^-24 per 3D transform on
+    the path from the inputs to the output and 4 per product around it, added as independent ones,
+    times 2 for bands whose result is smaller than its terms.  7e-7 to 1.5e-6."""
+    return 2.0 * 2.0 ** -24 * math.sqrt(transforms * (2.0 * math.log2(n[0] * n[1] * n[2]) + 4.0))
 
 
 def per_band_rel(sys_, nb, got, ref):

@@ -2,9 +2,7 @@
 
 Every compiled grid size, TC and BITC, both precisions, ragged bands with an empty k; then bases whose
 spans go past half the grid, where sums of basis vectors wrap.  FP64 within 1e-10 relative.  FP32-split
-per band within rounding(n): about 4 log2 N + 8 roundings of 2^-24 lie on the path from the inputs to
-the output (two 3D transforms at about two a butterfly level, the products, the tables), independent
-ones add as a square root, and a factor 2 covers bands whose result is smaller than its terms.
+per band within the rounding bound of its path (fp32_rounding).
 
 The precision test holds FP32-split to what the reference's formula gives in 32 bits: with
 K = k - q + G, the products are K_d (chi* d_d phi_j) and (K_d u) rho, so rounding is relative to K p.
@@ -22,20 +20,16 @@ import scipy.fft
 from oracle import oracle as O
 from tc_amd import system as S
 from tc_amd import tcx
-from test_gpu_hf2x import per_band_rel
+from test_gpu_hf2x import fp32_rounding, per_band_rel
 
 pytestmark = pytest.mark.gpu
-
-
-def rounding(n):
-    return 2.0 * 2.0 ** -24 * math.sqrt(4.0 * math.log2(n[0] * n[1] * n[2]) + 8.0)
 
 
 def check(engine, sys_, nb, seed):
     engine.load_system(sys_)
     _, phi = S.applied_bands(sys_, nb=nb, seed=seed)
     ref = O.Oracle(sys_).tc2x(nb, phi)
-    for prec, tol in ((tcx.PREC_FP64, 1e-10), (tcx.PREC_FP32, rounding(sys_.n))):
+    for prec, tol in ((tcx.PREC_FP64, 1e-10), (tcx.PREC_FP32, fp32_rounding(sys_.n))):
         got = engine.tc2x(nb, phi, precision=prec)
         rel = per_band_rel(sys_, nb, got, ref).max()
         print(sys_.name, "precision", prec, f"per-band rel max {rel:.3e} (bound {tol:.1e})", flush=True)
