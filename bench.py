@@ -56,6 +56,14 @@ def read_traffic(name, pairs_per_launch):
     return float(entry["bytes_per_pair"]) * pairs_per_launch
 
 
+def record_bytes_per_pair(values, channels=1):
+    """FP32 bytes of pair records that the three passes of one pair move: the first writes `values`
+    complex values per channel, the middle one reads and writes them, the last one reads them.  The
+    orbital grids that a pass reads besides are shared by the pairs of a launch and come from cache
+    for the most part (counters: profiles/), so they do not count as HBM bytes."""
+    return [8.0 * channels * values * w for w in (1, 2, 1)]
+
+
 def cpu_model():
     """Model name of the host CPU (first /proc/cpuinfo entry), or None."""
     try:
@@ -298,13 +306,11 @@ def main():
     dom = int(np.argmax(ms[:3]))
     avg_ms = ms[dom] / max(1, launches[dom])
     pairs_per_launch = kpairs[dom] / max(1, launches[dom])
-    # FP32 complex values per pair: A reads phi_qi and writes the record's support columns, Z reads
-    # and writes them, C reads them and phi_qi
     n_rec = eng.record_columns("hf2x") * sys_.n[2]
-    words = [N + n_rec, 2 * n_rec, n_rec + N]
-    bytes_per_launch = 8.0 * words[dom] * pairs_per_launch
+    rec_bytes = record_bytes_per_pair(n_rec)
+    bytes_per_launch = rec_bytes[dom] * pairs_per_launch
     achieved = bytes_per_launch / (avg_ms * 1e-3) / 1e9
-    pipeline_gbs = 8.0 * sum(words) * pairs_per_step / (ms_per_step * 1e-3) / 1e9
+    pipeline_gbs = sum(rec_bytes) * pairs_per_step / (ms_per_step * 1e-3) / 1e9
     traffic = read_traffic(CLASS_NAMES[dom], pairs_per_launch)
 
     ceiling = copy_ceiling(eng)
@@ -376,12 +382,12 @@ def main():
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
             "kernel": CLASS_NAMES[dom], "avg_launch_ms": avg_ms, "pairs_per_launch": pairs_per_launch,
-            "algorithmic_bytes_per_launch": bytes_per_launch,
+            "record_bytes_per_launch": bytes_per_launch,
             "copy_ceiling_GBps": ceiling, "frac_of_copy_ceiling": achieved / ceiling,
         },
         "cpu_baseline": cpu,
         "pipeline": {
-            "algorithmic_GBps": pipeline_gbs, "record_values_per_pair": n_rec, "frac_of_hbm": pipeline_gbs / HBM_PEAK_GBS,
+            "record_GBps": pipeline_gbs, "record_values_per_pair": n_rec, "frac_of_hbm": pipeline_gbs / HBM_PEAK_GBS,
             "class_ms_per_step": {CLASS_NAMES[c]: float(ms[c]) / args.steps for c in range(4)},
             "launches_per_step": {CLASS_NAMES[c]: int(launches[c]) // args.steps for c in range(4)},
         },
@@ -671,9 +677,7 @@ def bench_tc_legs(eng, log, tc_steps):
             of its dominant pass; one FP64 apply after a warm-up; energy and per-band errors;
       tc3a3b3b4b6, tc3a2a4b2b5: FP32-split first apply (occupied-set work included), repeated
             apply (occupied-set q-sums reused), FP64 first apply; energy errors.
-    Algorithmic bytes per tc2x pair and pass (N points, 8 B per FP32 complex value): pass A
-    reads chi_qi and writes 4 record channels (5 N 8 B), pass B reads and writes 4 channels
-    (8 N 8 B), pass C reads 4 channels and the 4 grids of phi_qi and grad phi_qi (8 N 8 B)."""
+    The tc2x roofline counts the bytes of its four record channels (record_bytes_per_pair)."""
     from tc_amd import energy as E
     from tc_amd import system as S
     from tc_amd import tcx
@@ -732,22 +736,22 @@ def bench_tc_legs(eng, log, tc_steps):
     h64 = d_out.download(np.complex128)
     e32 = E.term_energy(sys_, h32, 2, left=True)
     e64 = E.term_energy(sys_, h64, 2, left=True)
-    words = [5, 8, 8]   # grid values moved per pair in passes A, B, C
+    rec_bytes = record_bytes_per_pair(N, 4)
     dom = int(np.argmax(ms[:3]))
     avg_ms = ms[dom] / max(1, launches[dom])
     ppl = kpairs[dom] / max(1, launches[dom])
-    bpl = words[dom] * N * 8 * ppl
+    bpl = rec_bytes[dom] * ppl
     fp32_s = float(np.median(t32))
     res["tc2x"] = {
         "fp32_ms": fp32_s * 1e3, "fp64_ms": t64 * 1e3, "fp32_over_fp64": t64 / fp32_s,
         "fp32_pairs_per_s": pairs / fp32_s, "E_fp64_Ha": [float(e64.real), float(e64.imag)],
         "dE_Ha": float(abs(e32 - e64)), "per_band_rel_max": per_band(h32, h64),
-        "pipeline_algorithmic_GBps_21NBc": 21 * N * 8 * pairs / fp32_s / 1e9,
+        "pipeline_record_GBps": sum(rec_bytes) * pairs / fp32_s / 1e9,
         "roofline": {"bound": "hbm", "achieved": bpl / (avg_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": bpl / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
                      "traffic": read_traffic("tc2x_" + Z_FIRST_NAMES[dom], ppl),
                      "kernel": "tc2x_" + Z_FIRST_NAMES[dom], "avg_launch_ms": avg_ms, "pairs_per_launch": ppl,
-                     "algorithmic_bytes_per_launch": bpl},
+                     "record_bytes_per_launch": bpl},
         "class_ms_per_apply": {Z_FIRST_NAMES[c]: float(ms[c]) / tc_steps for c in range(4)},
     }
     # ---- three-body exchange terms
