@@ -384,9 +384,10 @@ int tcx_memset_zero(tcx_context *ctx, void *ptr, unsigned long long bytes);
  * then the xy planes, then z back), 1 plane-first (xy planes, then z pencils, then xy back;
  * FP32-split only: the pair records then hold only the (kx, ky) columns inside the pair
  * density's G-space support, about two thirds of them at 40^3), -1 automatic (the default:
- * plane-first in FP32-split, except in the applies of tcx_davidson).  No counterpart in the
- * reference, whose hf2x runs full 3D FFTs (src/calc_hamiltonian_hf2x.cpp:123-135);
- * the two orders agree to rounding. */
+ * plane-first in FP32-split, except inside tcx_davidson and tcx_grad_exchange, which return
+ * numbers at the level of rounding: the phases of eigenvectors, the imaginary part of E_x).  No
+ * counterpart in the reference, whose hf2x runs full 3D FFTs
+ * (src/calc_hamiltonian_hf2x.cpp:123-135); the two orders agree to rounding. */
 int tcx_set_pipeline_order(tcx_context *ctx, int term, int order);
 
 /* Mean number of (kx, ky) columns per plane of the pair records of the last apply of

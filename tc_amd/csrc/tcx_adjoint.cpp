@@ -77,7 +77,8 @@ void Context::grad_x(double* grad, double* energy, int prec)
     std::vector<cd> phi(ncoef), h(ncoef, cd(0.0));
     if (ncoef) {
         TCX_HIP_CHECK(hipMemcpy(phi.data(), d_phi_occ.p, ncoef * 16, hipMemcpyDeviceToHost));
-        hf2x(nocc.data(), reinterpret_cast<const double*>(phi.data()), reinterpret_cast<double*>(h.data()), prec, 0);
+        hf2x(nocc.data(), reinterpret_cast<const double*>(phi.data()), reinterpret_cast<double*>(h.data()), prec,
+             kFlagZFirst);
     }
     const cd e = half_energy(phi, h, occ_coef, nocc, npw, fill, num_kpoints);
     energy[0] = e.real();

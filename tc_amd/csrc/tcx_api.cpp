@@ -593,7 +593,7 @@ void Context::ensure_gradR(int prec)
 // Z-first: enough targets that pass C issues kAutoTargetWaves wavefronts, then as many
 // sources as kAutoBufferGrids pair grids allow (channels = grids per pair record: 1 for
 // hf2x, 4 for tc2x).
-void Context::resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources) const
+void Context::resolve_shape(int term, bool plane_first, long& tc, long& sc, long ntargets, long nsources) const
 {
     constexpr long kAutoTargetWaves = 8192, kAutoBufferGrids = 8192;
     constexpr long kXcds = 8, kL2Share = 3 << 20, kRounds = 4, kRecordBytes = (long)4 << 30;
@@ -603,7 +603,7 @@ void Context::resolve_shape(int term, int prec, long& tc, long& sc, long ntarget
     const long waves_per_target = ((long)geo.n1 * geo.n2 + 31) / 32;
     tc = (kAutoTargetWaves + waves_per_target - 1) / waves_per_target;
     sc = 0;
-    if (term == 0 && use_plane_first(prec)) {
+    if (plane_first) {
         const long grid_bytes = (long)N * 8;
         const PlaneShape ps = plane_shape(geo.n1);
         auto even = [](long n, long most) { return (n + (n + most - 1) / most - 1) / ((n + most - 1) / most); };
@@ -725,12 +725,12 @@ const BandJobs& Context::get_band_jobs(const std::vector<int>& nb)
 }
 
 // term 0: hf2x, 1: tc2x, kPlanJobs: the per-band jobs without the band pairs
-const Plan& Context::get_plan(const std::vector<int>& nb, int term, int prec)
+const Plan& Context::get_plan(const std::vector<int>& nb, int term, bool plane_first)
 {
     long nt = 0;
     for (int k = 0; k < nk; ++k) nt += nb[k];
     long tc = 0, sc = 0;
-    if (term != kPlanJobs) resolve_shape(term, prec, tc, sc, nt, n_occ);
+    if (term != kPlanJobs) resolve_shape(term, plane_first, tc, sc, nt, n_occ);
     auto key = std::make_tuple(nb, tc, sc);
     auto it = plans.find(key);
     if (it != plans.end()) return it->second;
@@ -853,7 +853,8 @@ void Context::hf2x(const int* nb_, const double* phi, double* out, int prec, uns
 {
     check_apply_args(nb_, phi, out, prec);
     std::vector<int> nb(nb_, nb_ + nk);
-    const Plan& P = get_plan(nb, 0, prec);
+    const bool plane_first = use_plane_first(prec, flags);
+    const Plan& P = get_plan(nb, 0, plane_first);
     ApplyIO io = begin_apply(nb_, phi, out, flags, P);
     if (P.n_app > 0) {
         ensure_occR(prec);
@@ -861,7 +862,7 @@ void Context::hf2x(const int* nb_, const double* phi, double* out, int prec, uns
         d_appR.ensure((size_t)P.n_app * N * es);
         timed(3, 0, [&] { orbitals_to_real(io.phi, (const OrbEntry*)P.d_appjobs.p, P.n_app, prec, d_appR.p); });
         begin_W(P.n_app);
-        if (use_plane_first(prec)) {
+        if (plane_first) {
             hf2x_plane_first(P);
             double factor = -4.0 * kPiHost / (num_kpoints * volume);  // two_body_factor, hf2x.cpp:29-30
             if (nspin == 1) factor /= 2.0;
@@ -1051,7 +1052,7 @@ int tcx_set_density(tcx_context* ctx, const double* density)
 
 int tcx_hf2x(tcx_context* ctx, const int* nb, const double* phi, double* h2phi, int precision, unsigned flags)
 {
-    return guarded(ctx, [&] { ctx->impl.hf2x(nb, phi, h2phi, precision, flags); });
+    return guarded(ctx, [&] { ctx->impl.hf2x(nb, phi, h2phi, precision, flags & ~kFlagZFirst); });
 }
 
 int tcx_set_zero_weight_kpoints(tcx_context* ctx, const double* kweight, const double* sum_of_kvaux,
@@ -1110,7 +1111,7 @@ int tcx_tc2h(tcx_context* ctx, const int* nb, const double* phi, double* h2phi, 
 int tcx_apply_all(tcx_context* ctx, const int* nb, const double* phi, double* h1phi, double* h2phi, double* h3phi,
                   int precision, unsigned flags)
 {
-    return guarded(ctx, [&] { ctx->impl.apply_all(nb, phi, h1phi, h2phi, h3phi, precision, flags); });
+    return guarded(ctx, [&] { ctx->impl.apply_all(nb, phi, h1phi, h2phi, h3phi, precision, flags & ~kFlagZFirst); });
 }
 
 int tcx_davidson(tcx_context* ctx, const int* nb, double* phi, double* phi_left, double* eig, double* energies,

@@ -347,16 +347,13 @@ void Context::davidson(const int* nb_, double* phi_d, double* phi_left_d, double
         launch_dv_copy(d64(left ? dVL[cur] : dV[cur]), dl(kVoff), di(kFirst), d64(dIn), dl(kCoff), nullptr, di(kCnt),
                        max_cnt, di(kNpw), max_npw, nk, stream);
         if (left) hermitian_conj();
-        in_davidson = true;
         try {
             apply_all(it(kCnt), d64(dIn), d64(dO[0]), d64(dO[1]), uses3 ? d64(dO[2]) : nullptr, prec,
-                      TCX_FLAG_DEVICE_PTRS);
+                      TCX_FLAG_DEVICE_PTRS | kFlagZFirst);
         } catch (...) {
-            in_davidson = false;
             if (left) hermitian_conj();
             throw;
         }
-        in_davidson = false;
         if (left) hermitian_conj();
         for (int n = 0; n < nH; ++n)
             launch_dv_copy(d64(dO[n]), dl(kCoff), nullptr, d64(left ? dHLV[n] : dHV[n]), dl(kVoff), di(kFirst),

@@ -25,13 +25,15 @@ int centered_host(int i, int n) { return i <= n / 2 ? i : i - n; }
 
 // Automatic order: plane-first in FP32-split (40^3, 4x4x4 k, 16 bands: 428 ms per apply against
 // 535), z-first in FP64 (36^3: 18.2 ms of pair passes against 18.4; the FP64 line transforms of
-// pass C take every register).  The Davidson's applies keep z-first: its eigensolver takes the
-// phases of eigenvectors from rounding-level entries, so another order of the same sums would
-// flip the signs of some returned bands.
-bool Context::use_plane_first(int prec) const
+// pass C take every register).  Calls that return numbers at the level of rounding keep the z-first
+// sums that have given them so far (kFlagZFirst): tcx_davidson, whose eigensolver takes the phases of
+// the eigenvectors from rounding-level entries, so another order flips the signs of some returned
+// bands, and tcx_grad_exchange, whose imaginary part of E_x is rounding alone (0 by Hermiticity).
+// hf2x is the only term with two orders; TC and BITC applies hold none of it.
+bool Context::use_plane_first(int prec, unsigned flags) const
 {
     if (prec != TCX_PREC_FP32 || hf2x_order == 0) return false;
-    return hf2x_order == 1 || !in_davidson;
+    return hf2x_order == 1 || !(flags & kFlagZFirst);
 }
 
 // One column set for every (k, q): per kx, the hull of the ky differences of all bases.

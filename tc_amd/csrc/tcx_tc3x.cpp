@@ -740,7 +740,7 @@ void Context::apply_all(const int* nb_, const double* phi, double* h1, double* h
         if (bytes) TCX_HIP_CHECK(hipMemcpyAsync(base, phi, bytes, hipMemcpyHostToDevice, stream));
         double* dev[3];
         for (int n = 0; n < nout; ++n) dev[n] = (double*)(base + (size_t)(1 + n) * slot);
-        apply_all(nb_, (const double*)base, dev[0], dev[1], tc ? dev[2] : nullptr, prec, TCX_FLAG_DEVICE_PTRS);
+        apply_all(nb_, (const double*)base, dev[0], dev[1], tc ? dev[2] : nullptr, prec, flags | TCX_FLAG_DEVICE_PTRS);
         for (int n = 0; n < nout; ++n)
             if (bytes) TCX_HIP_CHECK(hipMemcpyAsync(outs[n], dev[n], bytes, hipMemcpyDeviceToHost, stream));
         TCX_HIP_CHECK(hipStreamSynchronize(stream));

@@ -64,6 +64,10 @@ struct TablePiece {
 // for all tables of a plan) and points the views at them.
 void upload_tables(DBuf& buf, std::initializer_list<TablePiece> pieces);
 
+// Beside the TCX_FLAG_* of a term call, set inside the library only: automatic pass order z-first
+// (Context::use_plane_first).
+constexpr unsigned kFlagZFirst = 1u << 31;
+
 // One launch of the pair pipeline.
 struct Launch {
     int pair0 = 0, npairs = 0;      // slice of Plan::pairs; slot p of the pair buffer = pair0 + p
@@ -193,8 +197,7 @@ struct Context {
     long shape_sources[3] = {0, 0, 0};
     int hf2x_order = -1;          // -1 automatic, 0 z-first, 1 plane-first (FP32)
     double hf2x_record_cols = 0;  // (kx, ky) columns per plane of the last hf2x apply's records
-    bool in_davidson = false;     // an apply of tcx_davidson runs (use_plane_first)
-    bool use_plane_first(int prec) const;
+    bool use_plane_first(int prec, unsigned flags = 0) const;
     // support columns of the pair records and whether differences of basis vectors stay inside the
     // grid; both belong to the basis (tcx_set_basis), their tables lie behind d_gindex's indices
     PlaneCols cols{};
@@ -328,9 +331,9 @@ struct Context {
     void jastrow_kernels(int s1, int s2, long long n, const double* G2, double* uk, double* v);
     void ensure_density();
 
-    void resolve_shape(int term, int prec, long& tc, long& sc, long ntargets, long nsources) const;
+    void resolve_shape(int term, bool plane_first, long& tc, long& sc, long ntargets, long nsources) const;
     static constexpr int kPlanJobs = -1;
-    const Plan& get_plan(const std::vector<int>& nb, int term, int prec = 0);
+    const Plan& get_plan(const std::vector<int>& nb, int term, bool plane_first = false);
     void check_apply_args(const int* nb, const double* phi, const double* out, int prec);
     ApplyIO begin_apply(const int* nb, const double* phi, double* out, unsigned flags, const Plan& P);
     void end_apply(const ApplyIO& io);

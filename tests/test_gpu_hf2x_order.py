@@ -101,3 +101,22 @@ def test_plane_first_wrapping_columns(engine, gw, mesh):
         assert per_band_rel(sys_, nb, out[order], ref).max() <= fp32_rounding(sys_.n)
     engine.set_pipeline_order("hf2x", -1)
     assert per_band_rel(sys_, nb, out[1], out[0]).max() <= 1e-6
+
+
+def test_calls_that_return_rounding_keep_z_first(engine):
+    """Phases of Davidson's eigenvectors and Im E_x are set by rounding, so with the automatic order
+    they come from the z-first sums, bit for bit; an order that was asked for is taken."""
+    sys_ = S.tiny_system(method="HF", n=(16, 16, 16), kmesh=(2, 2, 1), nbands=3, nocc=3, seed_stream=540)
+    engine.load_system(sys_)
+    nb, phi = S.applied_bands(sys_, nb=np.array([3, 3, 2, 3], np.int32), seed=541)
+    eig = np.zeros(int(nb.sum()), complex)
+    out = {}
+    for order in (-1, 0, 1):
+        engine.set_pipeline_order("hf2x", order)
+        e, g = engine.grad_exchange(precision=tcx.PREC_FP32)
+        out[order] = [np.array([e]), g, engine.davidson(nb, phi, eig, precision=tcx.PREC_FP32)[0]]
+    engine.set_pipeline_order("hf2x", -1)
+    for a, b, c in zip(out[-1], out[0], out[1]):
+        assert np.array_equal(a, b)
+        assert not np.array_equal(a, c)
+    assert abs(out[1][0][0].real - out[0][0][0].real) <= 1e-6 * abs(out[0][0][0].real)
