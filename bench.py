@@ -578,14 +578,16 @@ def bench_batched(log, replays):
 def bench_davidson(eng, log):
     """One block-Davidson update of the 16 occupied bands of the HF 4x4x4 k, 40^3 cell
     (host pointers in and out, as TC++ calls it): wall time against one apply of
-    calc_hamiltonian::all on the same bands; the difference over the two applies the
-    Davidson makes is the cost of its device-resident FP64 subspace algebra."""
+    calc_hamiltonian::all on the same bands, in the z-first order that the Davidson's applies
+    take; the difference over the two applies the Davidson makes is the cost of its
+    device-resident FP64 subspace algebra."""
     from tc_amd import system as S
     from tc_amd import tcx
 
     sys_ = S.fcc_hf_40()
     eng.load_system(sys_)
     nb, phi = sys_.nocc.copy(), sys_.phi_occ
+    eng.set_pipeline_order("hf2x", 0)
     h1, h2, _ = eng.apply_all(nb, phi, precision=tcx.PREC_FP32)  # warm-up (plans, workspaces)
     d_phi = eng.to_device(phi)
     d_h = [eng.device_buffer(phi.nbytes) for _ in range(2)]
@@ -597,6 +599,7 @@ def bench_davidson(eng, log):
     eng.synchronize()
     t_apply = time.perf_counter() - t0
     eng._check(st, "apply_all")
+    eng.set_pipeline_order("hf2x", -1)
     for b in [d_phi] + d_h:
         b.free()
     bo = sys_.band_offsets(nb)
